@@ -354,6 +354,7 @@ void GpuSolver::upload_forest(const std::vector<const Octree*>& trees)
     ghat_if_.clear();
     ghat_lap32_.clear();
     ghat_if32_.clear();
+    if_iv_.clear();
     uploaded_ = true;
 }
 
@@ -510,6 +511,7 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
     auto      T = [&](int s) { return (mtgt_[s] >> idx) & 1ULL; };
 
 
+    p.npairs = 0;
     p.antrp.clear();
     p.antrp.resize(L + 1);
     p.intrp.clear();
@@ -572,11 +574,14 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
         }
     }
 
+    // Trees whose targets the separable sums serve (neighbour-only passes).
+    std::vector<char> sep(ntrees_, 0);
+    if (nbonly) build_separable(p, sep);
+
     // pairs per target and sibling groups per level
     std::vector<char> is_src(nb_, 0);
     std::vector<int>  inv;
     p.mac.clear();
-    p.npairs = 0;
     const int lmin = nbonly ? L : 0;
     for (int lam = L; lam >= lmin; --lam)
     {
@@ -591,7 +596,7 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
         long                                   pairs_here = 0;
         for (int t = lvl_begin_[lam]; t < lvl_begin_[lam + 1]; ++t)
         {
-            if (!T(t)) continue;
+            if (!T(t) || sep[tree_of_[t]]) continue;
             std::vector<int> srcs;
             if (lam == L)
                 for (int i = 0; i < 27; ++i)
@@ -787,6 +792,75 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
     p.zero_t.upload(zt);
 }
 
+// The entries of launch::if_separable for one neighbour-only pass.  A tree
+// qualifies when every source that a target lists sits at the neighbour
+// slot's own offset (Morton keys that wrap at coarse levels list blocks
+// elsewhere, or twice; such a tree keeps the spectral path).  The scratch
+// positions are the blocks' places at x, y offsets of the targets that have a
+// source below, at or above them: at most three per source, which is what
+// the source spectra's array, their scratch, holds in either precision.
+void GpuSolver::build_separable(PassPlan& p, std::vector<char>& done)
+{
+    const int L = p.L;
+    auto      S = [&](int s) { return (msrc_[s] >> p.idx) & 1ULL; };
+    auto      T = [&](int s) { return (mtgt_[s] >> p.idx) & 1ULL; };
+    auto      place = [&](int tree, int x, int y, int z) {  // coordinates are below 2^15; -1 and 2^15 are places too
+        return (static_cast<uint64_t>(tree) << 48) | (static_cast<uint64_t>(x + 1) << 32) |
+               (static_cast<uint64_t>(y + 1) << 16) | static_cast<uint64_t>(z + 1);
+    };
+    std::unordered_map<uint64_t, int> source;
+    std::fill(done.begin(), done.end(), 1);
+    if (ntrees_ > 65535 || L > 14)
+    {
+        std::fill(done.begin(), done.end(), 0);
+        return;
+    }
+    for (int s = lvl_begin_[L]; s < lvl_begin_[L + 1]; ++s)
+        if (S(s)) source[place(tree_of_[s], coord_[3 * s], coord_[3 * s + 1], coord_[3 * s + 2])] = s;
+    auto find = [&](int tree, int x, int y, int z) {
+        const auto it = source.find(place(tree, x, y, z));
+        return it == source.end() ? -1 : it->second;
+    };
+    for (int t = lvl_begin_[L]; t < lvl_begin_[L + 1]; ++t)
+    {
+        if (!T(t) || !done[tree_of_[t]]) continue;
+        for (int i = 0; i < 27; ++i)
+        {
+            const int s = neighbor_[27 * t + i], o[3] = {i % 3 - 1, (i / 3) % 3 - 1, i / 9 - 1};
+            bool      same = (s >= 0 && S(s) ? s : -1) ==
+                        find(tree_of_[t], coord_[3 * t] + o[0], coord_[3 * t + 1] + o[1], coord_[3 * t + 2] + o[2]);
+            for (int d = 0; d < 3 && s >= 0; ++d)
+                if (S(s) && bbase_[3 * s + d] - bbase_[3 * t + d] != o[d] * e_) same = false;
+            if (!same) done[tree_of_[t]] = 0;
+        }
+    }
+    std::unordered_map<uint64_t, int> pos;
+    std::vector<int>                  zent, tent;
+    for (int t = lvl_begin_[L]; t < lvl_begin_[L + 1]; ++t)
+    {
+        const int tree = tree_of_[t];
+        if (!T(t) || !done[tree]) continue;
+        int  e[10] = {t, -1, -1, -1, -1, -1, -1, -1, -1, -1};
+        bool any = false;
+        for (int i = 0; i < 9; ++i)
+        {
+            const int x = coord_[3 * t] + i % 3 - 1, y = coord_[3 * t + 1] + i / 3 - 1, z = coord_[3 * t + 2];
+            const int b[3] = {find(tree, x, y, z - 1), find(tree, x, y, z), find(tree, x, y, z + 1)};
+            for (int s : b) p.npairs += s >= 0 ? 1 : 0;
+            if (b[0] < 0 && b[1] < 0 && b[2] < 0) continue;
+            const auto it = pos.emplace(place(tree, x, y, z), static_cast<int>(zent.size() / 3));
+            if (it.second) zent.insert(zent.end(), b, b + 3);
+            e[1 + i] = it.first->second;
+            any = true;
+        }
+        if (any) tent.insert(tent.end(), e, e + 10);
+    }
+    p.sep_z.upload(zent);
+    p.sep_t.upload(tent);
+    const size_t room = static_cast<size_t>(nb_) * nf_;  // doubles of one component's FP32 source spectra
+    if (zent.size() / 3 * launch::if_mid_size(n_) > room) throw std::logic_error("separable pass: scratch positions");
+}
+
 PassPlan& GpuSolver::pass(int L, int nl, bool nbonly)
 {
     return pass_idx(L, fmm_mask_idx_gen(MASK_AMR2AMR, L - base_level_, nl), nbonly);
@@ -832,19 +906,28 @@ double2* GpuSolver::ghat_if(double alpha)
     if (gen_sample_.n < (size_t)nsample) gen_sample_.alloc(nsample);
     if (gen_a_.n < (size_t)nleg) gen_a_.alloc(nleg);
     if (gen_b_.n < (size_t)nleg) gen_b_.alloc(nleg);
-    const int           kmax = 3 * e_ + n_;
-    std::vector<double> iv(kmax + 1);
-    scaled_bessel_i(2.0 * alpha, kmax, iv.data());
-    sync();  // the previous iv upload may still be read
-    d_iv_.upload(iv);
+    const int         kmax = 3 * e_ + n_;
+    const double*     iv = if_iv(alpha);
     DevArray<double2> g;
     g.alloc(static_cast<size_t>(343) * nf_);
-    launch::lgf_spectra(stream_, n_, 1, 0, nullptr, 0, d_iv_.p, kmax, gen_sample_.p, gen_a_.p, gen_b_.p, g.p);
+    launch::lgf_spectra(stream_, n_, 1, 0, nullptr, 0, iv, kmax, gen_sample_.p, gen_a_.p, gen_b_.p, g.p);
     IBLGF_HIP(hipGetLastError());
     sync();
     auto* ptr = g.p;
     ghat_if_[alpha] = std::move(g);
     return ptr;
+}
+
+const double* GpuSolver::if_iv(double alpha)
+{
+    auto it = if_iv_.find(alpha);
+    if (it != if_iv_.end()) return it->second.p;
+    const int           kmax = 3 * e_ + n_;
+    std::vector<double> iv(kmax + 1);
+    scaled_bessel_i(2.0 * alpha, kmax, iv.data());
+    DevArray<double> a;
+    a.upload(iv);
+    return (if_iv_[alpha] = std::move(a)).p;
 }
 
 const void* GpuSolver::ghat(bool laplace, int d, double alpha)
@@ -894,8 +977,10 @@ void GpuSolver::prepare_if(double alpha_base)
 {
     for (int l = base_level_; l < depth_; ++l)
     {
-        for (int nl = 0; nl < 2; ++nl) pass(l, nl, true);
-        ghat(false, 0, alpha_base * std::pow(4.0, l - base_level_));
+        const double alpha = alpha_base * std::pow(4.0, l - base_level_);
+        if_iv(alpha);
+        for (int nl = 0; nl < 2; ++nl)
+            if (!pass(l, nl, true).mac.empty()) ghat(false, 0, alpha);
     }
     sync();
 }
@@ -914,6 +999,15 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
     // Kernel spectra first: building one launches work on the solver stream.
     std::vector<const void*> gh(p.mac.size());
     for (size_t i = 0; i < p.mac.size(); ++i) gh[i] = ghat(laplace, p.mac[i].d, alpha);
+    if (p.sep_t.size() > 0)
+    {
+        const double* iv = if_iv(alpha);
+        timer_.begin(stream_);
+        launch::if_separable(stream_, n_, wp_.src, static_cast<double*>(wp_.sspec), wp_.tgt, p.sep_z.p,
+            p.sep_z.size() / 3, p.sep_t.p, p.sep_t.size() / 10, iv, b, b.sstride);
+        timer_.end(stream_, KC_OTHER, 0);
+    }
+    if (p.neighbor_only && p.mac.empty()) return;
     // Two chains over disjoint blocks.  Fine (solver stream): the level-L
     // sources' forward transform, read in place from the solve's source array
     // with their rings as zero (Fmm::apply copies interiors into zeroed
@@ -1327,7 +1421,7 @@ bool GpuSolver::prepared(bool laplace, double alpha_base) const
         for (int nl = 0; nl < 2; ++nl)
         {
             const auto it = passes_.find(pass_key(l, fmm_mask_idx_gen(MASK_AMR2AMR, l - base_level_, nl), !laplace));
-            if (it == passes_.end()) return false;
+            if (it == passes_.end() || (!laplace && !if_iv_.count(alpha))) return false;
             for (const auto& m : it->second->mac)
                 if (!has_ghat(laplace, m.d, alpha)) return false;
         }

@@ -78,6 +78,9 @@ struct PassPlan
     std::vector<DevArray<int>>       antrp;  // by level (parents)
     std::vector<DevArray<int>>       intrp;  // by level (parents at level)
     std::vector<MacLevelPlan>        mac;
+    // Neighbour-only passes: the targets summed directly (if_separable), and
+    // the source slots of its scratch positions.
+    DevArray<int>                    sep_z, sep_t;
     long                             npairs = 0;
     long                             ntransfer = 0;  // parent-child transfers (anterp + interp)
     long                             ntransfer_antrp = 0;
@@ -329,6 +332,8 @@ class GpuSolver
     PassPlan& pass_idx(int L, int idx, bool neighbor_only);
     static int pass_key(int L, int idx, bool neighbor_only) { return (L * 64 + idx) * 2 + (neighbor_only ? 1 : 0); }
     bool      has_ghat(bool laplace, int d, double alpha) const;
+    void      build_separable(PassPlan& p, std::vector<char>& done);
+    const double* if_iv(double alpha);
     const DevArray<int>& face_clean_list(int kind, int level, bool leaf_only);
     void      run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& b);
     void      lgf_batch_body(const int* src, const int* dst, int k);
@@ -418,10 +423,10 @@ class GpuSolver
     std::map<double, DevArray<double2>>      ghat_if_;
     std::map<int, DevArray<float2>>          ghat_lap32_;
     std::map<double, DevArray<float2>>       ghat_if32_;
+    std::map<double, DevArray<double>>       if_iv_;  // e^{-2 alpha} I_k(2 alpha), k <= 3 e + n
     int                                      precision_ = 0;
     DevArray<double>                         gen_sample_;
     DevArray<double2>                        gen_a_, gen_b_;
-    DevArray<double>                         d_iv_;
 
     // plans
     std::map<int, std::unique_ptr<PassPlan>> passes_;

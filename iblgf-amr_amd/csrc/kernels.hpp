@@ -154,6 +154,17 @@ void forward_dft_mfma(hipStream_t s, int n, int prec, const double* field, const
 void inverse_dft_mfma(hipStream_t s, int n, int prec, const float2* spec, const int* slots, int count,
     double* field, double scale, bool accumulate, const Batch& b = {});
 
+// One neighbour-only integrating-factor pass as separable sums
+// (if_separable.hip): dst[target] += every point's sum over the interiors of
+// the neighbour blocks.  zent[npos][3]: source slots below, at and above each
+// scratch position (-1: none); ent[ntgt][10]: target slot, then the scratch
+// positions at x, y offsets (ox + 1) + 3 (oy + 1) (-1: none); iv[k] =
+// e^{-2a} I_k(2a), k <= 2 (n - 2).  mid: scratch of if_mid_size(n) values per
+// position, mid_stride from one component's scratch to the next.
+constexpr long if_mid_size(int n) { return (long)n * (n - 2) * (n - 2); }
+void if_separable(hipStream_t s, int n, const double* src, double* mid, double* dst, const int* zent, int npos,
+    const int* ent, int ntgt, const double* iv, const Batch& b, long mid_stride);
+
 // Kernel spectra for the 343 offsets o in [-3,3]^3 at level difference d:
 // block[a] = K(step*(-o*e - (n-1) + a)), a in [0,P)^3, step = 2^d, then r2c.
 // kind 0: Laplace LGF (table g up to nmax, asymptotics beyond);
