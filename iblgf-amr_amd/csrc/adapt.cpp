@@ -63,12 +63,14 @@ int GpuSolver::readapt(const Octree& t, const int* fields, const int* mesh, cons
     auto lap32 = std::move(ghat_lap32_);
     auto lif32 = std::move(ghat_if32_);
     auto iv = std::move(if_iv_);
+    auto pg = std::move(par_ghat_);
     upload_tree(t);
     ghat_lap_ = std::move(lap);
     ghat_if_ = std::move(lif);
     ghat_lap32_ = std::move(lap32);
     ghat_if32_ = std::move(lif32);
     if_iv_ = std::move(iv);
+    par_ghat_ = std::move(pg);
     step_ready_ = false;  // the step's work fields were dropped with the old arrays
     // every field id again, at the new size
     fields_.clear();

@@ -286,6 +286,8 @@ void GpuSolver::upload_forest(const std::vector<const Octree*>& trees)
     fields_.clear();
     drop_graphs();
     work_ = Work{};
+    par_need_s_ = par_need_t_ = par_need_m_ = 0;
+    for (DevArray<double2>* a : {&par_sspec_, &par_tspec_, &par_mid_}) *a = DevArray<double2>{};
     reserve_components(1);
 
     // solver-level block lists
@@ -355,6 +357,7 @@ void GpuSolver::upload_forest(const std::vector<const Octree*>& trees)
     ghat_lap32_.clear();
     ghat_if32_.clear();
     if_iv_.clear();
+    par_ghat_ = DevArray<double2>{};
     uploaded_ = true;
 }
 
@@ -588,6 +591,7 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
         struct GroupBuild
         {
             MacGroup                            g;
+            int                                 tree, coord[3];  // the parent's
             std::vector<std::array<int, 3>>     ent;      // (slot, r, tmask)
             std::unordered_map<int, std::vector<int>> by_slot;
         };
@@ -611,7 +615,6 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
                     if (s >= 0 && S(s)) srcs.push_back(s);
                 }
             if (srcs.empty()) continue;
-            inv.push_back(t);
             // sibling groups are keyed by (tree, parent key): keys repeat across a forest
             const std::pair<int, uint64_t> pk(tree_of_[t], Morton::parent(key_[t]));
             auto                           it = gidx.find(pk);
@@ -621,6 +624,8 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
                 gi = static_cast<int>(gb.size());
                 gidx[pk] = gi;
                 GroupBuild b;
+                b.tree = tree_of_[t];
+                for (int d = 0; d < 3; ++d) b.coord[d] = coord_[3 * t + d] >> 1;
                 std::fill(b.g.tslot, b.g.tslot + 8, -1);
                 b.g.begin = b.g.count = b.g.nfull = 0;
                 gb.push_back(std::move(b));
@@ -667,16 +672,101 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
                     ids.push_back(static_cast<int>(gb[gi].ent.size()));
                     gb[gi].ent.push_back({s, rr, 1 << cb});
                 }
-                is_src[s] = 1;
                 ++pairs_here;
             }
         }
         if (gb.empty()) continue;
+        // Level-L groups of a tree whose every group sums over all source
+        // blocks of its region, once each, run by whole parents; their block
+        // entries are counted and not uploaded.
+        std::vector<char> whole(ntrees_, lam == L && !nbonly ? 1 : 0);
+        std::unordered_map<uint64_t, std::array<int, 8>> kids;  // source blocks by parent place
+        auto place = [](int tree, const int c[3]) {
+            return (static_cast<uint64_t>(tree) << 48) | (static_cast<uint64_t>(c[0] + 1) << 32) |
+                   (static_cast<uint64_t>(c[1] + 1) << 16) | static_cast<uint64_t>(c[2] + 1);
+        };
+        auto around = [](const GroupBuild& b, int o, int c[3]) {
+            c[0] = b.coord[0] + o % 3 - 1;
+            c[1] = b.coord[1] + (o / 3) % 3 - 1;
+            c[2] = b.coord[2] + o / 9 - 1;
+        };
+        if (lam == L && !nbonly)
+        {
+            if (ntrees_ > 65535 || L > 14) std::fill(whole.begin(), whole.end(), 0);  // places hold 16 bits each
+            for (int s = lvl_begin_[L]; s < lvl_begin_[L + 1]; ++s)
+                if (S(s))
+                {
+                    const int c[3] = {coord_[3 * s] >> 1, coord_[3 * s + 1] >> 1, coord_[3 * s + 2] >> 1};
+                    auto      it = kids.find(place(tree_of_[s], c));
+                    if (it == kids.end())
+                    {
+                        it = kids.emplace(place(tree_of_[s], c), std::array<int, 8>{}).first;
+                        it->second.fill(-1);
+                    }
+                    it->second[(coord_[3 * s] & 1) | (coord_[3 * s + 1] & 1) << 1 | (coord_[3 * s + 2] & 1) << 2] = s;
+                }
+            for (const auto& b : gb)
+            {
+                int gmask = 0, found = 0;
+                for (int c = 0; c < 8; ++c) gmask |= b.g.tslot[c] >= 0 ? 1 << c : 0;
+                for (const auto& en : b.ent)
+                    if (en[2] != gmask) whole[b.tree] = 0;
+                for (int o = 0; o < 27 && whole[b.tree]; ++o)
+                {
+                    int c[3];
+                    around(b, o, c);
+                    const auto it = kids.find(place(b.tree, c));
+                    if (it == kids.end()) continue;
+                    for (int s : it->second)
+                        if (s >= 0)
+                        {
+                            ++found;
+                            if (!b.by_slot.count(s)) whole[b.tree] = 0;
+                        }
+                }
+                if (found != static_cast<int>(b.ent.size())) whole[b.tree] = 0;
+            }
+        }
         std::vector<MacGroup> groups;
         std::vector<MacSrc>   srcs;
         long                  m_nfull = 0, m_pairs_full = 0, m_pop[8] = {};
+        std::vector<int>      psrc, ptgt, pbegin(1, 0), pent;  // as ParentPass
+        std::unordered_map<uint64_t, int> pidx;
+        long                  pairs_parents = 0, entries_parents = 0;
         for (auto& b : gb)
         {
+            long gpairs = 0;
+            for (const auto& en : b.ent) gpairs += __builtin_popcount(static_cast<unsigned>(en[2]));
+            for (int c = 0; c < 8; ++c)
+                if (b.g.tslot[c] >= 0)
+                {
+                    if (whole[b.tree]) ++p.par_ninv;
+                    else
+                        inv.push_back(b.g.tslot[c]);
+                }
+            if (whole[b.tree])
+            {
+                ptgt.insert(ptgt.end(), b.g.tslot, b.g.tslot + 8);
+                for (int o = 0; o < 27; ++o)
+                {
+                    int c[3];
+                    around(b, o, c);
+                    const auto it = kids.find(place(b.tree, c));
+                    if (it == kids.end()) continue;
+                    const auto at = pidx.emplace(it->first, static_cast<int>(psrc.size() / 8));
+                    if (at.second)
+                    {
+                        psrc.insert(psrc.end(), it->second.begin(), it->second.end());
+                        for (int s : it->second) p.par_nfwd += s >= 0 ? 1 : 0;
+                    }
+                    pent.push_back(at.first->second * 32 + o);
+                }
+                pbegin.push_back(static_cast<int>(pent.size()));
+                pairs_parents += gpairs;
+                entries_parents += static_cast<long>(b.ent.size());
+                continue;
+            }
+            for (const auto& en : b.ent) is_src[en[0]] = 1;
             b.g.begin = static_cast<int>(srcs.size());
             std::vector<MacSrc> loc;
             for (auto& en : b.ent)
@@ -713,6 +803,26 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
             b.g.count = static_cast<int>(loc.size());
             groups.push_back(b.g);
         }
+        if (!ptgt.empty())
+        {
+            p.npar_src = static_cast<int>(psrc.size() / 8);
+            p.npar_tgt = static_cast<int>(ptgt.size() / 8);
+            p.par_src.upload(psrc);
+            p.par_tgt.upload(ptgt);
+            p.par_begin.upload(pbegin);
+            p.par_ent.upload(pent);
+            p.par_npairs = p.par_stats.npairs = p.par_stats.pairs_full = pairs_parents;
+            p.par_stats.nentries = p.par_stats.nfull = entries_parents;
+            const ParentGeo g = launch::parent_geo(n_);
+            const size_t    nf = g.NF;
+            par_need_s_ = std::max(par_need_s_, p.npar_src * nf);
+            par_need_t_ = std::max(par_need_t_, p.npar_tgt * nf);
+            par_need_m_ = std::max({par_need_m_, static_cast<size_t>(p.npar_src) * g.H * g.M * g.M,
+                static_cast<size_t>(p.npar_tgt) * g.H * g.W * g.W});
+            p.npairs += pairs_parents;
+            pairs_here -= pairs_parents;
+        }
+        if (groups.empty()) continue;
         MacLevelPlan m;
         m.lambda = lam;
         m.d = L - lam;
@@ -790,6 +900,12 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
         for (int s = lvl_begin_[l]; s < lvl_begin_[l + 1]; ++s)
             if (T(s) && !written[s]) zt.push_back(s);
     p.zero_t.upload(zt);
+    // a pass whose sources and targets are all at level L has no second chain to fork and join
+    p.coarse = !nbonly && L > 0 &&
+               (p.zero_s.size() || p.zero_t.size() || p.nfwd_coarse || p.ninv_top < p.inv.size());
+    for (const auto& e : p.antrp) p.coarse = p.coarse || e.size();
+    for (const auto& e : p.intrp) p.coarse = p.coarse || e.size();
+    for (const auto& m : p.mac) p.coarse = p.coarse || m.lambda != L;
 }
 
 // The entries of launch::if_separable for one neighbour-only pass.  A tree
@@ -969,8 +1085,53 @@ void GpuSolver::prepare_laplace()
         {
             PassPlan& p = pass(l, nl, false);
             for (auto& m : p.mac) ghat(true, m.d, 0.0);
+            if (p.npar_tgt > 0) parent_ghat();
         }
+    reserve_parents();
     sync();
+}
+
+// Kernel spectra of the whole-parent transforms (level difference
+// 0, FP64; functions of the block size only).
+const double2* GpuSolver::parent_ghat()
+{
+    if (par_ghat_.n > 0) return par_ghat_.p;
+    const ParentGeo  g = launch::parent_geo(n_);
+    const size_t     nf = static_cast<size_t>(g.H) * g.P * g.P;
+    DevArray<double> sample;
+    sample.alloc(static_cast<size_t>(14) * g.P * g.P * g.P);
+    DevArray<double2> a, b, gh;
+    a.alloc(14 * nf);
+    b.alloc(14 * nf);
+    gh.alloc(14 * static_cast<size_t>(g.NF));
+    launch::parent_sample(stream_, n_, d_lgf_table_.p, lgf_nmax_, sample.p);
+    launch::parent_spectra(stream_, n_, sample.p, a.p, b.p, gh.p);
+    IBLGF_HIP(hipGetLastError());
+    sync();  // the scratch is released on return
+    par_ghat_ = std::move(gh);
+    return par_ghat_.p;
+}
+
+// Scratch of the whole-parent transforms for every pass built so far and the
+// component count of the work arrays.
+void GpuSolver::reserve_parents()
+{
+    const size_t k = static_cast<size_t>(work_.k);
+    if (par_sspec_.n >= par_need_s_ * k && par_tspec_.n >= par_need_t_ * k && par_mid_.n >= par_need_m_ * k) return;
+    sync();         // passes in flight still use the old arrays
+    drop_graphs();  // captured graphs point at the old arrays
+    if (par_sspec_.n < par_need_s_ * k) par_sspec_.alloc(par_need_s_ * k);
+    if (par_tspec_.n < par_need_t_ * k) par_tspec_.alloc(par_need_t_ * k);
+    if (par_mid_.n < par_need_m_ * k) par_mid_.alloc(par_need_m_ * k);
+}
+
+void GpuSolver::run_parents(PassPlan& p, double scale, const Batch& b)
+{
+    const double2* g = parent_ghat();
+    reserve_parents();
+    const ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt, g,
+        par_sspec_.p, par_tspec_.p, par_mid_.p};
+    launch::parent_pass(stream_, n_, precision_, pp, wp_.src, wp_.tgt, scale, b);
 }
 
 void GpuSolver::prepare_if(double alpha_base)
@@ -1017,7 +1178,7 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
     // interpolation down to level L-1.  They join before the last
     // interpolation, which adds into the level-L targets.  Issued in an order
     // that is also valid on one stream.
-    const bool  coarse = !p.neighbor_only && L > 0;
+    const bool  coarse = p.coarse;
     const bool  two = coarse && concurrent_;
     hipStream_t A = stream_, B = two ? side_ : stream_;
     if (two)
@@ -1039,6 +1200,12 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
                 m_nli_anterp_.p, false, b, top);
         }
         timer_.end(B, KC_TRANSFER, p.ntransfer_antrp * b.k);
+    }
+    if (p.npar_tgt > 0)
+    {
+        timer_.begin(A);
+        run_parents(p, scale, b);
+        timer_.end(A, KC_MAC, p.par_npairs * b.k);
     }
     const int nfine = static_cast<int>(p.fwd.size()) - p.nfwd_coarse;
     timer_.begin(A);
@@ -1424,6 +1591,9 @@ bool GpuSolver::prepared(bool laplace, double alpha_base) const
             if (it == passes_.end() || (!laplace && !if_iv_.count(alpha))) return false;
             for (const auto& m : it->second->mac)
                 if (!has_ghat(laplace, m.d, alpha)) return false;
+            if (it->second->npar_tgt > 0 && (par_ghat_.n == 0 || par_sspec_.n < par_need_s_ ||
+                                                par_tspec_.n < par_need_t_ || par_mid_.n < par_need_m_))
+                return false;
         }
     }
     return true;
@@ -1703,10 +1873,13 @@ SolveCounts GpuSolver::lgf_counts() const
         const PassPlan& p = *kv.second;
         if (p.neighbor_only || p.idx < 15 || p.idx >= 30) continue;  // Laplace AMR2AMR passes only
         c.passes += 1;
-        c.n_src += p.fwd.size();
-        c.n_tgt += p.inv.size();
+        c.n_src += p.fwd.size() + p.par_nfwd;
+        c.n_tgt += p.inv.size() + p.par_ninv;
         c.n_pair += p.npairs;
         c.n_transfer += p.ntransfer;
+        c.n_entry += p.par_stats.nentries;
+        c.n_entry_full += p.par_stats.nfull;
+        c.n_pair_full += p.par_stats.pairs_full;
         for (const auto& m : p.mac)
         {
             c.n_entry += m.nentries;

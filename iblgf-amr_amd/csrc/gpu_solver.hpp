@@ -72,6 +72,7 @@ struct PassPlan
 {
     int                              L = 0, nl = 0, idx = 0;
     bool                             neighbor_only = false;
+    bool                             coarse = false;  // there is work at levels below L
     DevArray<int>                    zero_s, zero_t, fwd, inv;
     int                              ninv_top = 0;     // inv starts with the level-L targets
     int                              nfwd_coarse = 0;  // fwd ends with the level-L sources
@@ -81,6 +82,13 @@ struct PassPlan
     // Neighbour-only passes: the targets summed directly (if_separable), and
     // the source slots of its scratch positions.
     DevArray<int>                    sep_z, sep_t;
+    // Laplace passes: the level-L sums by transforms of whole parents
+    // (parent_fft.hip), the blocks that take that path, and the statistics of
+    // their pairs (the entries a block-wise plan would have).
+    DevArray<int>                    par_src, par_tgt, par_begin, par_ent;
+    int                              npar_src = 0, npar_tgt = 0;
+    long                             par_nfwd = 0, par_ninv = 0, par_npairs = 0;
+    MacLevelPlan                     par_stats;
     long                             npairs = 0;
     long                             ntransfer = 0;  // parent-child transfers (anterp + interp)
     long                             ntransfer_antrp = 0;
@@ -333,6 +341,9 @@ class GpuSolver
     static int pass_key(int L, int idx, bool neighbor_only) { return (L * 64 + idx) * 2 + (neighbor_only ? 1 : 0); }
     bool      has_ghat(bool laplace, int d, double alpha) const;
     void      build_separable(PassPlan& p, std::vector<char>& done);
+    void      reserve_parents();
+    const double2* parent_ghat();
+    void      run_parents(PassPlan& p, double scale, const Batch& b);
     const double* if_iv(double alpha);
     const DevArray<int>& face_clean_list(int kind, int level, bool leaf_only);
     void      run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& b);
@@ -413,6 +424,13 @@ class GpuSolver
         void*   tspec = nullptr;
     };
     WorkPtrs wp_;
+    // Scratch of the whole-parent transforms, for the largest pass built and
+    // work_.k components: spectra of source and target parents and the
+    // half-transformed columns between the kernels.  A context's own, so an
+    // allocation-free solve finds it after prepare.
+    DevArray<double2> par_sspec_, par_tspec_, par_mid_;
+    size_t            par_need_s_ = 0, par_need_t_ = 0, par_need_m_ = 0;  // of one component
+    DevArray<double2> par_ghat_;
     bool                                          graphs_ = false;
     std::map<std::vector<int64_t>, hipGraphExec_t> graph_cache_;
 

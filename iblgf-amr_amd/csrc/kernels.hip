@@ -1177,6 +1177,27 @@ __global__ __launch_bounds__(kThreads) void k_lgf_sample(int kind, int d, const 
     out[q] = v;
 }
 
+// The Laplace kernel between two parents of M = 2 E points a side at offset o
+// (13 .. 26 of 27; the first 13 are mirror images): out[o - 13][z][y][x] at
+// point difference m = target - source, cyclic of length P.
+__global__ __launch_bounds__(kThreads) void k_parent_sample(
+    int M, int P, const double* __restrict__ g, int nmax, double* __restrict__ out)
+{
+    const long PPP = (long)P * P * P, q = (long)blockIdx.x * kThreads + threadIdx.x;
+    if (q >= 14 * PPP) return;
+    const int  o = 13 + (int)(q / PPP);
+    int        m[3] = {(int)(q % P), (int)((q / P) % P), (int)((q / ((long)P * P)) % P)};
+    const int  off[3] = {o % 3 - 1, (o / 3) % 3 - 1, o / 9 - 1};
+    bool       used = true;
+    for (int d = 0; d < 3; ++d)
+    {
+        if (m[d] > M) m[d] -= P;
+        used = used && m[d] >= -M;  // a length above 2 M + 1 leaves differences that no pair has
+        m[d] -= M * off[d];
+    }
+    out[q] = used ? lgf_value(g, nmax, m[0], m[1], m[2]) : 0.0;
+}
+
 // x leg: in[o][z][y][x] real -> out[o][z][y][kx]
 template<int N>
 __global__ __launch_bounds__(kThreads) void k_leg_x(const double* __restrict__ in, double2* __restrict__ out)
@@ -1558,6 +1579,12 @@ void spectral_mac(hipStream_t s, int n, int prec, const MacGroup* groups, int ng
     if (ngroups > 0)
         dispatch_n<RunMac>(n, s, prec, groups, ngroups, srcs, rowoff, olist, nused, compact, ghat, sspec, tspec, b,
             b.mac_policy == 2 ? queue : nullptr);
+}
+void parent_sample(hipStream_t s, int n, const double* g, int nmax, double* sample)
+{
+    const ParentGeo p = parent_geo(n);
+    hipLaunchKernelGGL(
+        k_parent_sample, dim3(grid1(14L * p.P * p.P * p.P)), dim3(kThreads), 0, s, p.M, p.P, g, nmax, sample);
 }
 void to_float2(hipStream_t s, const double2* in, float2* out, long n)
 {

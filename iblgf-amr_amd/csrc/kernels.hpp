@@ -87,6 +87,33 @@ constexpr int kPrecFp64 = 0, kPrecMixed = 1, kPrecBf16x3 = 2, kPrecF16x3 = 3, kP
 constexpr int kPrecF16x3Forward = 6;
 constexpr bool prec_mfma(int p) { return p >= kPrecBf16x3 && p <= kPrecI8x4; }
 
+// The finest level of one Laplace pass by transforms of whole parents
+// (parent_fft.hip).  Sizes at block size n: M source and W target points a
+// side of a parent, transform length P, H = P / 2 + 1 stored z frequencies;
+// a spectrum has H P P values.
+struct ParentGeo
+{
+    int M, W, P, H, NF;
+};
+// src_child[nsrc][8], tgt_child[ntgt][8]: block slots of the children (-1:
+// not a source / target); entries begin[t] .. begin[t + 1] of target t: source
+// parent * 32 + offset (ox + 1) + 3 (oy + 1) + 9 (oz + 1) of the source.
+// ghat: 14 spectra of parent_spectra (offsets 13 to 26).  Scratch for k components: sspec and
+// tspec a spectrum per source / target parent (FP64, or FP32 with prec > 0),
+// mid H values a column for the larger of nsrc M M and ntgt W W columns.
+struct ParentPass
+{
+    const int*     src_child;
+    const int*     tgt_child;
+    const int*     begin;
+    const int*     entries;
+    int            nsrc, ntgt;
+    const double2* ghat;
+    void*          sspec;
+    void*          tspec;
+    double2*       mid;
+};
+
 namespace launch {
 
 bool supported_n(int n);
@@ -164,6 +191,14 @@ void inverse_dft_mfma(hipStream_t s, int n, int prec, const float2* spec, const 
 constexpr long if_mid_size(int n) { return (long)n * (n - 2) * (n - 2); }
 void if_separable(hipStream_t s, int n, const double* src, double* mid, double* dst, const int* zent, int npos,
     const int* ent, int ntgt, const double* iv, const Batch& b, long mid_stride);
+
+ParentGeo parent_geo(int n);
+// dst[target block] += scale * (every point's sum over the sources' interiors).
+void parent_pass(hipStream_t s, int n, int prec, const ParentPass& p, const double* src, double* dst, double scale,
+    const Batch& b);
+// sample: 14 P^3 values; a, b: scratch of 14 H P P values each; ghat: 14 NF.
+void parent_sample(hipStream_t s, int n, const double* g, int nmax, double* sample);
+void parent_spectra(hipStream_t s, int n, const double* sample, double2* a, double2* b, double2* ghat);
 
 // Kernel spectra for the 343 offsets o in [-3,3]^3 at level difference d:
 // block[a] = K(step*(-o*e - (n-1) + a)), a in [0,P)^3, step = 2^d, then r2c.
