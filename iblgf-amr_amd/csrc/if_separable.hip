@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kSepThreads) void k_if_z(const double* __restrict__
     const int* __restrict__ zent, int npos, const double* __restrict__ iv, long fcs, long mcs)
 {
     constexpr int E = N - 2, EE = E * E, NN = N * N, N3 = N * NN;
-    const int     q = blockIdx.x * kSepThreads + threadIdx.x;
+    const int     q = xcd_item(blockIdx.x, gridDim.x) * kSepThreads + threadIdx.x;
     const int     pos = q / EE, col = q - pos * EE;
     if (pos >= npos) return;
     src += blockIdx.y * fcs + NN + (col / E + 1) * N + col % E + 1;
@@ -78,14 +78,16 @@ constexpr int sep_threads() { return (N * N + 63) / 64 * 64; }
 
 template<int N>
 __global__ __launch_bounds__(sep_threads<N>()) void k_if_yx(const double* __restrict__ mid, double* __restrict__ dst,
-    const int* __restrict__ entries, const double* __restrict__ iv, long mcs, long fcs)
+    const int* __restrict__ entries, int ntgt, const double* __restrict__ iv, long mcs, long fcs)
 {
     constexpr int E = N - 2, EE = E * E, NN = N * N, N3 = N * NN, T = sep_threads<N>();
     // odd rows: the y leg's 64-bit stores, a stride of one row apart, meet different banks
     constexpr int     ROW = NN + 1;
     constexpr int     kBuf = E * ROW > N3 ? E * ROW : N3;
     __shared__ double buf[kBuf];
-    const int*        ent = entries + 10 * blockIdx.x;
+    const int         item = xcd_item(blockIdx.x, gridDim.x);
+    if (item >= ntgt) return;  // the whole workgroup
+    const int*        ent = entries + 10 * item;
     const int         l = threadIdx.x, z = l / E, x = l - z * E;
     mid += blockIdx.y * mcs + z * EE + x;
     double out[N];
@@ -133,9 +135,10 @@ void run(hipStream_t s, const double* src, double* mid, double* dst, const int* 
     int ntgt, const double* iv, const Batch& b, long mcs)
 {
     const long cols = (long)npos * (N - 2) * (N - 2);
-    hipLaunchKernelGGL(k_if_z<N>, dim3((unsigned)((cols + kSepThreads - 1) / kSepThreads), b.k), dim3(kSepThreads), 0,
+    hipLaunchKernelGGL(k_if_z<N>, dim3(xcd_grid((cols + kSepThreads - 1) / kSepThreads), b.k), dim3(kSepThreads), 0,
         s, src, mid, zent, npos, iv, b.fstride, mcs);
-    hipLaunchKernelGGL(k_if_yx<N>, dim3(ntgt, b.k), dim3(sep_threads<N>()), 0, s, mid, dst, ent, iv, mcs, b.fstride);
+    hipLaunchKernelGGL(k_if_yx<N>, dim3(xcd_grid(ntgt), b.k), dim3(sep_threads<N>()), 0, s, mid, dst, ent, ntgt, iv, mcs,
+        b.fstride);
 }
 
 }  // namespace

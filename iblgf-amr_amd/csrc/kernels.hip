@@ -6,7 +6,7 @@
 //   spectral_mac                simd_prod_complex_add over all (source, target)
 //                               pairs of Fmm::compute_influence_field,
 //                               include/iblgf/fmm/fmm.hpp:988-1027, 1167-1195
-//   transfer_gather / _scatter  Nli::nli_antrp_node / nli_intrp_node,
+//   transfer (gather, scatter)  Nli::nli_antrp_node / nli_intrp_node,
 //                               include/iblgf/fmm/fmm_nli.hpp:101-247; cell_center_nli
 //                               include/iblgf/interpolation/cell_center_nli_intrp.hpp:337-420, 591-674
 //   buffer_exchange             halo fill, include/iblgf/domain/mpi/haloCommunicator.hpp:67-128
@@ -130,190 +130,172 @@ __global__ __launch_bounds__(kThreads) void k_axpy(
 }
 
 // ---------------------------------------------------------------------------
-// Separable 3-leg transfer: out[k][j][i] = sum Kz[k][c] Ky[j][b] Kx[i][a] in[c][b][a]
-// Every leg is line-per-thread: a thread takes a whole line (N points along
-// the leg's axis) into registers and writes its N outputs; the matrix row
-// index is uniform across the workgroup, so matrix reads from LDS are
-// broadcasts.  The x leg reads the input block from global memory, the y leg
-// runs in place in the one LDS buffer, the z leg writes global memory.
+// Separable 3-leg transfer: out[k][j][i] = sum Kz[k][c] Ky[j][b] Kx[i][a] in[c][b][a],
+// summed over a parent's children or applied to one parent.  A workgroup
+// computes KZ of a block's N output planes: the z leg runs first, from global
+// memory (a thread per column, neighbouring threads next to each other in x),
+// and what is left, y and x, stays within those planes in LDS.  So a block is
+// N / KZ independent workgroups, and a parent's children meet as soon as they
+// can: the two of a column in the z leg, four sums of them in the y leg, two
+// in the x leg (14 leg applications where child after child takes 24).  A
+// thread takes a whole line of inputs into registers; the matrix index is the
+// same for a whole wave, so the matrix is read through the scalar unit and
+// multiplies from scalar registers.  Waits for memory bound it: the 17 gathers
+// and 20 scatters of a 4290-block solve of 16^3 cells take 0.42 and 0.45 ms
+// (FP64, one stream; a workgroup per block, child after child: 0.89 and 0.66).
 // ---------------------------------------------------------------------------
-// One thread per line of a leg: the n^2 = 324 lines of an 18^3 block fit one
-// round of 384 threads.
-constexpr int kTransferThreads = 384;
+// KZ planes a workgroup, OG outputs of a line a thread (divisors of N).  A
+// gather has four times the z columns: half the outputs a thread, twice the
+// threads, so that they are two rounds of loads.
+template<int N, bool GATHER> struct TransferShape;
+template<> struct TransferShape<8, false> { static constexpr int KZ = 4, OG = 4; };
+template<> struct TransferShape<10, false> { static constexpr int KZ = 5, OG = 5; };
+template<> struct TransferShape<12, false> { static constexpr int KZ = 4, OG = 4; };
+template<> struct TransferShape<16, false> { static constexpr int KZ = 4, OG = 4; };
+template<> struct TransferShape<18, false> { static constexpr int KZ = 6, OG = 6; };
+template<> struct TransferShape<8, true> { static constexpr int KZ = 4, OG = 2; };
+template<> struct TransferShape<10, true> { static constexpr int KZ = 5, OG = 2; };
+template<> struct TransferShape<12, true> { static constexpr int KZ = 4, OG = 2; };
+template<> struct TransferShape<16, true> { static constexpr int KZ = 4, OG = 2; };
+template<> struct TransferShape<18, true> { static constexpr int KZ = 6, OG = 3; };
 
-template<int N>
-struct TransferLds
+template<int N, bool GATHER>
+struct TransferGeo
 {
-    double buf[Geo<N>::N3];
+    static constexpr int KZ = TransferShape<N, GATHER>::KZ, OG = TransferShape<N, GATHER>::OG;
+    static constexpr int NN = N * N, PARTS = N / KZ, LINES = KZ * N;
+    static constexpr int NG = N / OG;                          // output ranges of a line, one per wave
+    static constexpr int T = 64 * NG * ((LINES + 63) / 64);    // and 64 lines of the planes per wave
 };
 
-// out[base + o*stride] = sum_a K[o][a] v[a].  K is read from global memory at
-// indices uniform across the workgroup, so the reads are scalar loads and
-// the FMAs take the matrix from scalar registers.
-template<int N>
-__device__ inline void line_apply(const double (&v)[N], const double* __restrict__ K, double* out, int base,
-    int stride)
+// acc[o] += sum_a K[o][a] v[a] for rows of N values at mats + at.  The rows are
+// loaded here, at each use (the offset is opaque): kept from one use to the
+// next they would not fit the scalar registers.
+template<int N, int OUTS>
+__device__ inline void rows_apply(const double (&v)[N], const double* __restrict__ mats, int at, double (&acc)[OUTS])
 {
-#pragma unroll 2
-    for (int o = 0; o < N; ++o)
+    asm volatile("" : "+s"(at));
+    const double* K = mats + at;
+#pragma unroll
+    for (int o = 0; o < OUTS; ++o)
     {
         double s = 0.0;
 #pragma unroll
         for (int a = 0; a < N; ++a) s = fma(K[o * N + a], v[a], s);
-        out[base + o * stride] = s;
+        acc[o] += s;
     }
 }
 
-// x and y legs: global block -> LDS buffer (x), then y in place.  `next`
-// (optional): a block the workgroup reads next; once this block's loads are
-// issued and consumed, each thread touches one 128-byte line of it, so its
-// lines are on their way while the y and z legs run on LDS.  The touched value
-// is held in `pend` and folded into `touch` only after the following block's
-// loads are issued, so no wait is placed on it before then.
-template<int N>
-__device__ inline void transfer_xy(const double* __restrict__ in, TransferLds<N>& L, const double* __restrict__ Kx,
-    const double* __restrict__ Ky, bool ring0 = false, const double* __restrict__ next = nullptr,
-    double* pend = nullptr, double* touch = nullptr)
-{
-    static_assert(N * N <= kTransferThreads, "one line per thread");
-    const int l = threadIdx.x;
-    if (l < N * N)
-    {
-        // ring0: the input block's boundary ring is read as zero
-        const int  lz = l / N, ly = l - lz * N;
-        const bool zl = ring0 && (lz == 0 || ly == 0 || lz == N - 1 || ly == N - 1);
-        double     v[N];
-#pragma unroll
-        for (int a = 0; a < N; ++a) v[a] = in[l * N + a];  // loaded unconditionally, then masked (no branches)
-        if (touch) *touch += *pend;
-        if (ring0)
-        {
-#pragma unroll
-            for (int a = 0; a < N; ++a) v[a] = (zl || a == 0 || a == N - 1) ? 0.0 : v[a];
-        }
-        line_apply<N>(v, Kx, L.buf, l * N, 1);
-    }
-    constexpr int kLines = (Geo<N>::N3 * 8 + 127) / 128;
-    if (next && l < kLines) *pend = next[l * 16];
-    __syncthreads();
-    if (l < N * N)
-    {
-        const int base = (l / N) * N * N + (l % N);
-        double    v[N];
-#pragma unroll
-        for (int b = 0; b < N; ++b) v[b] = L.buf[base + b * N];
-        line_apply<N>(v, Ky, L.buf, base, N);  // the thread owns this line
-    }
-    __syncthreads();
-}
-
-// z leg of line l = (j, i): acc[k] (+)= sum_c Kz[k][c] t2[c][j][i]
-template<int N>
-__device__ inline void leg_z_acc(const double* t2, const double* __restrict__ Kz, double (&acc)[N])
-{
-    const int l = threadIdx.x;
-    double    v[N];
-#pragma unroll
-    for (int c = 0; c < N; ++c) v[c] = t2[c * N * N + l];
-#pragma unroll
-    for (int k = 0; k < N; ++k)  // fully unrolled: acc stays in registers
-    {
-        double s = 0.0;
-#pragma unroll
-        for (int c = 0; c < N; ++c) s = fma(Kz[k * N + c], v[c], s);
-        acc[k] += s;
-    }
-}
-
-// Side matrix of one leg.  mesh < 0: mats is [2][N*N] (by the child's bit on
+// Offset of the side matrix of one leg in mats.  mesh < 0: mats is [2][N*N] (by the child's bit on
 // the leg's axis), the FMM's Lagrange operators.  mesh >= 0: mats is
 // [2 relative positions][2][N*N], the cell-centred level transfers, with the
 // relative position on each axis set by the field's mesh type
 // (cell_center_nli_intrp.hpp:599-618): cell 1 on every axis; face component
 // fi 0 on axis fi, 1 elsewhere; edge component fi 1 on axis fi, 0 elsewhere.
 template<int N>
-__device__ inline const double* side_mat(const double* mats, int mesh, int fi, int axis, int bit)
+__device__ inline int side_mat(int mesh, int fi, int axis, int bit)
 {
     constexpr int NN = N * N;
-    if (mesh < 0) return mats + bit * NN;
+    if (mesh < 0) return bit * NN;
     const int rel = mesh == 1 ? (axis == fi ? 0 : 1) : (mesh == 2 ? (axis == fi ? 1 : 0) : 1);
-    return mats + (rel * 2 + bit) * NN;
+    return (rel * 2 + bit) * NN;
 }
 
-// dst[parent] (=|+=) sum over listed children of K(child); one workgroup per
-// parent, the children's contributions summed in registers in child order and
-// written to (added into) the parent once, every point of it (deterministic).
-template<int N>
-__global__ __launch_bounds__(kTransferThreads) void k_transfer_gather(
-    const double* __restrict__ src, double* __restrict__ dst, const int* __restrict__ entries, int count,
-    const double* __restrict__ mats, int accumulate, int ring0, long cs, int mesh, int comp0)
+// GATHER: dst[parent] (=|+=) sum over the listed children of K(child), entries
+// {parent, child[8]}; otherwise dst[child] (=|+=) K(src[parent]), entries
+// {child, parent, child id}.  ring0: the inputs' boundary rings are read as zero.
+template<int N, bool GATHER>
+__global__ __launch_bounds__((TransferGeo<N, GATHER>::T)) void k_transfer(const double* __restrict__ src,
+    double* __restrict__ dst, const int* __restrict__ entries, int count, const double* __restrict__ mats,
+    int accumulate, int ring0, long cs, int mesh, int comp0)
 {
-    constexpr int N3 = Geo<N>::N3;
-    __shared__ TransferLds<N> L;
-    const int e = blockIdx.x;
-    if (e >= count) return;
+    using G = TransferGeo<N, GATHER>;
+    constexpr int     KZ = G::KZ, OG = G::OG, NN = G::NN, N3 = Geo<N>::N3, NX = GATHER ? 2 : 1;
+    __shared__ double buf[NX * NX * KZ * NN];  // [x and y side][plane][y][x]
+    const int         item = xcd_item(blockIdx.x, gridDim.x);
+    if (item >= count * G::PARTS) return;
+    const int         e = item / G::PARTS, k0 = (item - e * G::PARTS) * KZ;
+    const int         fi = (comp0 + (int)blockIdx.y) % 3;
+    const int*        ent = entries + (GATHER ? 9 : 3) * e;
+    const int         id = GATHER ? 0 : ent[2];  // sides of the one transfer
     src += blockIdx.y * cs;
-    dst += blockIdx.y * cs;
-    const int  fi = (comp0 + (int)blockIdx.y) % 3;
-    const int* ent = entries + 9 * e;
-    double     acc[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) acc[k] = 0.0;
-    bool   first = true;
-    double touch = 0.0, pend = 0.0;
-    for (int c = 0; c < 8; ++c)
+    dst += blockIdx.y * cs + (size_t)ent[0] * N3 + k0 * NN;
+    for (int it = threadIdx.x; it < NX * NX * NN; it += G::T)
     {
-        const int ch = ent[1 + c];
-        if (ch < 0) continue;  // uniform across the workgroup
-        if (!first) __syncthreads();  // previous z leg done with the buffer
-        first = false;
-        int nx = -1;  // the next listed child, touched ahead of its x leg
-        for (int d = c + 1; d < 8 && nx < 0; ++d) nx = ent[1 + d];
-        transfer_xy<N>(src + (size_t)ch * N3, L, side_mat<N>(mats, mesh, fi, 0, c & 1),
-            side_mat<N>(mats, mesh, fi, 1, (c >> 1) & 1), ring0, nx >= 0 ? src + (size_t)nx * N3 : nullptr, &pend,
-            &touch);
-        if (threadIdx.x < N * N) leg_z_acc<N>(L.buf, side_mat<N>(mats, mesh, fi, 2, (c >> 2) & 1), acc);
-    }
-    asm volatile("" ::"v"(touch + pend));  // the touch loads are kept, their value unused
-    if (threadIdx.x < N * N)
-    {
-        double* out = dst + (size_t)ent[0] * N3 + threadIdx.x;
+        const int  xy = it / NN, col = it - xy * NN, y = col / N, x = col - y * N;
+        const bool edge = ring0 && (x == 0 || y == 0 || x == N - 1 || y == N - 1);
+        double     acc[KZ];
 #pragma unroll
-        for (int k = 0; k < N; ++k) out[k * N * N] = accumulate ? out[k * N * N] + acc[k] : acc[k];
-    }
-}
-
-// dst[entry.child] (=|+=) K(src[entry.parent])
-template<int N>
-__global__ __launch_bounds__(kTransferThreads) void k_transfer_scatter(
-    const double* __restrict__ src, double* __restrict__ dst, const int* __restrict__ entries, int count,
-    const double* __restrict__ mats, int accumulate, long cs, int mesh, int comp0)
-{
-    constexpr int N3 = Geo<N>::N3;
-    __shared__ TransferLds<N> L;
-    const int e = blockIdx.x;
-    if (e >= count) return;
-    src += blockIdx.y * cs;
-    dst += blockIdx.y * cs;
-    const int fi = (comp0 + (int)blockIdx.y) % 3;
-    const int child = entries[3 * e], parent = entries[3 * e + 1], c = entries[3 * e + 2];
-    transfer_xy<N>(src + (size_t)parent * N3, L, side_mat<N>(mats, mesh, fi, 0, c & 1),
-        side_mat<N>(mats, mesh, fi, 1, (c >> 1) & 1));
-    if (threadIdx.x < N * N)
-    {
-        double acc[N];
-#pragma unroll
-        for (int k = 0; k < N; ++k) acc[k] = 0.0;
-        leg_z_acc<N>(L.buf, side_mat<N>(mats, mesh, fi, 2, (c >> 2) & 1), acc);
-        double* out = dst + (size_t)child * N3 + threadIdx.x;
-#pragma unroll
-        for (int k = 0; k < N; ++k)
+        for (int k = 0; k < KZ; ++k) acc[k] = 0.0;
+#pragma unroll 1
+        for (int cz = 0; cz < NX; ++cz)  // (two uses of a matrix side by side spill scalar registers)
         {
-            if (accumulate) out[k * N * N] += acc[k];
-            else
-                out[k * N * N] = acc[k];
+            const int in = GATHER ? ent[1 + xy + 4 * cz] : ent[1];
+            if (in < 0 || edge) continue;
+            const double* p = src + (size_t)in * N3 + col;
+            double        v[N];
+#pragma unroll
+            for (int c = 0; c < N; ++c) v[c] = p[c * NN];
+            if (ring0) v[0] = v[N - 1] = 0.0;
+            rows_apply<N, KZ>(v, mats, side_mat<N>(mesh, fi, 2, GATHER ? cz : (id >> 2) & 1) + k0 * N, acc);
+        }
+#pragma unroll
+        for (int k = 0; k < KZ; ++k) buf[(xy * KZ + k) * NN + col] = acc[k];
+    }
+    __syncthreads();
+    const int  wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), o0 = (wave % G::NG) * OG;
+    const int  line = (wave / G::NG) * 64 + (threadIdx.x & 63), k = line / N, l = line - k * N;
+    const bool on = line < G::LINES;
+    double     out[NX][OG];
+#pragma unroll
+    for (int cx = 0; cx < NX; ++cx)
+#pragma unroll
+        for (int o = 0; o < OG; ++o) out[cx][o] = 0.0;
+    if (on)
+    {
+#pragma unroll
+        for (int cx = 0; cx < NX; ++cx)
+#pragma unroll 1
+            for (int cy = 0; cy < NX; ++cy)
+            {
+                double v[N];
+#pragma unroll
+                for (int b = 0; b < N; ++b) v[b] = buf[((cx + 2 * cy) * KZ + k) * NN + b * N + l];
+                rows_apply<N, OG>(
+                    v, mats, side_mat<N>(mesh, fi, 1, GATHER ? cy : (id >> 1) & 1) + o0 * N, out[cx]);
+            }
+    }
+    __syncthreads();
+    if (on)
+    {
+#pragma unroll
+        for (int cx = 0; cx < NX; ++cx)
+#pragma unroll
+            for (int o = 0; o < OG; ++o) buf[(cx * KZ + k) * NN + (o0 + o) * N + l] = out[cx][o];
+    }
+    __syncthreads();
+    double res[OG];
+#pragma unroll
+    for (int o = 0; o < OG; ++o) res[o] = 0.0;
+    if (on)
+    {
+#pragma unroll 1
+        for (int cx = 0; cx < NX; ++cx)
+        {
+            double v[N];
+#pragma unroll
+            for (int a = 0; a < N; ++a) v[a] = buf[(cx * KZ + k) * NN + l * N + a];
+            rows_apply<N, OG>(v, mats, side_mat<N>(mesh, fi, 0, GATHER ? cx : id & 1) + o0 * N, res);
         }
     }
+    __syncthreads();
+    if (on)
+    {
+#pragma unroll
+        for (int o = 0; o < OG; ++o) buf[line * N + o0 + o] = res[o];
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < KZ * NN; q += G::T) dst[q] = accumulate ? dst[q] + buf[q] : buf[q];
 }
 
 // ---------------------------------------------------------------------------
@@ -1322,8 +1304,9 @@ template<int N> struct RunGather
     static void run(hipStream_t s, const double* src, double* dst, const int* e, int count, const double* m,
         int accumulate, int ring0, const Batch& b, int mesh)
     {
-        hipLaunchKernelGGL(k_transfer_gather<N>, dim3(count, b.k), dim3(kTransferThreads), 0, s, src, dst, e, count,
-            m, accumulate, ring0, b.fstride, mesh, b.comp0);
+        using G = TransferGeo<N, true>;
+        hipLaunchKernelGGL((k_transfer<N, true>), dim3(xcd_grid((long)count * G::PARTS), b.k), dim3(G::T), 0, s, src, dst,
+            e, count, m, accumulate, ring0, b.fstride, mesh, b.comp0);
     }
 };
 template<int N> struct RunScatter
@@ -1331,8 +1314,9 @@ template<int N> struct RunScatter
     static void run(hipStream_t s, const double* src, double* dst, const int* e, int count, const double* m, int acc,
         const Batch& b, int mesh)
     {
-        hipLaunchKernelGGL(k_transfer_scatter<N>, dim3(count, b.k), dim3(kTransferThreads), 0, s, src, dst, e, count,
-            m, acc, b.fstride, mesh, b.comp0);
+        using G = TransferGeo<N, false>;
+        hipLaunchKernelGGL((k_transfer<N, false>), dim3(xcd_grid((long)count * G::PARTS), b.k), dim3(G::T), 0, s, src, dst,
+            e, count, m, acc, 0, b.fstride, mesh, b.comp0);
     }
 };
 template<int N> struct RunHalo

@@ -114,6 +114,14 @@ struct ParentPass
     double2*       mid;
 };
 
+// Workgroups are dealt to the 8 XCDs round-robin (workgroup i of a launch to
+// XCD i mod 8).  Where neighbouring work items read the same blocks, XCD x
+// takes the x-th contiguous eighth of `items`, so that the blocks are in its
+// L2: a grid of xcd_grid(items) workgroups along x, workgroup b doing
+// xcd_item(b, gridDim.x), nothing at or past the item count.
+inline unsigned xcd_grid(long items) { return (unsigned)((items + 7) / 8 * 8); }
+__device__ inline int xcd_item(unsigned b, unsigned grid) { return (int)((b & 7) * (grid >> 3) + (b >> 3)); }
+
 namespace launch {
 
 bool supported_n(int n);
