@@ -94,3 +94,24 @@ def test_argument_errors():
         helm2d_convolve(t, t, t)  # source and target must differ
     with pytest.raises(ValueError):
         helm2d_table([0.5], 8, 8, t.float())
+
+
+@pytest.mark.parametrize("nx,ny", [(8, 32), (15, 18), (31, 9), (32, 8), (33, 40), (63, 5), (64, 17), (65, 33), (128, 2),
+                                   (129, 7), (256, 9), (257, 16), (511, 3), (512, 8)])
+def test_transformed_widths_match_oracle(nx, ny):
+    """Patches whose x direction is transformed: the edges of the transform lengths and of the target-row
+    groups, rows of very different size next to each other, a scale.  FP64 transforms of up to 1024 points and sums
+    over at most 65 536 products: 1e-12 of the field."""
+    print(f"case: transformed convolution of 3 modes on a {nx} x {ny} patch", flush=True)
+    cs = np.array([0.05, 0.7, 3.0])
+    rng = np.random.default_rng(nx * ny)
+    src = rng.standard_normal((3, ny, nx)) * 10.0 ** rng.integers(-3, 4, (3, ny, 1))
+    t = torch.empty((3, ny, nx), dtype=torch.float64, device="cuda")
+    helm2d_table(cs, nx, ny, t)
+    s = torch.from_numpy(src).cuda()
+    d = torch.full_like(s, float("nan"))
+    helm2d_convolve(t, s, d, 0.6)
+    got, tab = d.cpu().numpy(), t.cpu().numpy()
+    for k in range(3):
+        ref = O.helm2d_convolve(tab[k], src[k], 0.6)
+        assert np.linalg.norm(got[k] - ref) <= 1e-12 * np.linalg.norm(ref), k
