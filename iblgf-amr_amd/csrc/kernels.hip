@@ -60,33 +60,20 @@ __global__ __launch_bounds__(kThreads) void k_zero(double* f, const int* slots, 
 }
 
 template<int N, class TD, class TS>
-__device__ inline void copy_block_as(TD* d, const TS* s, int interior)
+__device__ inline void copy_block(TD* d, const TS* s, int interior)
 {
-    for (int q = threadIdx.x; q < Geo<N>::N3; q += kThreads)
-    {
-        bool ring = false;
-        if (interior)
-        {
-            const int i = q % N, j = (q / N) % N, k = q / (N * N);
-            ring = i == 0 || j == 0 || k == 0 || i == N - 1 || j == N - 1 || k == N - 1;
-        }
-        d[q] = ring ? TD(0) : static_cast<TD>(s[q]);
-    }
-}
-
-template<int N>
-__device__ inline void copy_block(double* d, const double* s, int interior)
-{
-    for (int q = threadIdx.x; q < Geo<N>::N3; q += kThreads)
-    {
-        bool ring = false;
-        if (interior)
-        {
-            const int i = q % N, j = (q / N) % N, k = q / (N * N);
-            ring = i == 0 || j == 0 || k == 0 || i == N - 1 || j == N - 1 || k == N - 1;
-        }
-        d[q] = ring ? 0.0 : s[q];
-    }
+    each_point<Geo<N>::N3, kThreads>(
+        [=](int q) {
+            bool ring = false;
+            if (interior)
+            {
+                const int i = q % N, j = (q / N) % N, k = q / (N * N);
+                ring = i == 0 || j == 0 || k == 0 || i == N - 1 || j == N - 1 || k == N - 1;
+            }
+            const TD v = static_cast<TD>(s[q]);
+            return ring ? TD(0) : v;
+        },
+        [=](int q, TD v) { d[q] = v; });
 }
 
 template<int N>
@@ -110,11 +97,11 @@ __global__ __launch_bounds__(kThreads) void k_copy_table(
     const bool   df = (dst.f32 >> c) & 1ull, sf = (src.f32 >> c) & 1ull;  // uniform per workgroup
     if (!df && !sf) copy_block<N>(dst.p[c] + off, src.p[c] + off, interior);
     else if (df && !sf)
-        copy_block_as<N>(reinterpret_cast<float*>(dst.p[c]) + off, src.p[c] + off, interior);
+        copy_block<N>(reinterpret_cast<float*>(dst.p[c]) + off, src.p[c] + off, interior);
     else if (!df && sf)
-        copy_block_as<N>(dst.p[c] + off, reinterpret_cast<const float*>(src.p[c]) + off, interior);
+        copy_block<N>(dst.p[c] + off, reinterpret_cast<const float*>(src.p[c]) + off, interior);
     else
-        copy_block_as<N>(reinterpret_cast<float*>(dst.p[c]) + off, reinterpret_cast<const float*>(src.p[c]) + off,
+        copy_block<N>(reinterpret_cast<float*>(dst.p[c]) + off, reinterpret_cast<const float*>(src.p[c]) + off,
             interior);
 }
 
@@ -126,7 +113,9 @@ __global__ __launch_bounds__(kThreads) void k_axpy(
     const int b = blockIdx.x;
     if (b >= count) return;
     const size_t off = blockIdx.y * cs + (size_t)slots[b] * Geo<N>::N3;
-    for (int q = threadIdx.x; q < Geo<N>::N3; q += kThreads) dst[off + q] += src[off + q] * a;
+    each_point<Geo<N>::N3, kThreads>([=](int q) {
+#pragma clang fp contract(off)
+        return dst[off + q] + src[off + q] * a; }, [=](int q, double v) { dst[off + q] = v; });
 }
 
 // ---------------------------------------------------------------------------
@@ -330,17 +319,28 @@ __global__ __launch_bounds__(kThreads) void k_buffer_exchange(
     if (b >= count) return;
     f += blockIdx.y * cs;
     const int s = slots[b];
-    for (int r = threadIdx.x; r < RING; r += kThreads)
+    // every value of the thread loaded before the first is stored
+    constexpr int R = (RING + kThreads - 1) / kThreads;
+    const int*    nbs = neighbor + 27 * s;
+    double*       blk = f + (size_t)s * N3;
+    double        v[R];
+    int           to[R];
+#pragma unroll
+    for (int u = 0; u < R; ++u)
     {
-        const int q = ring_point<N>(r);
+        const int q = ring_point<N>(min((int)threadIdx.x + u * kThreads, RING - 1));
         const int i = q % N, j = (q / N) % N, k = q / (N * N);
         const int dx = i == 0 ? -1 : (i == N - 1 ? 1 : 0);
         const int dy = j == 0 ? -1 : (j == N - 1 ? 1 : 0);
         const int dz = k == 0 ? -1 : (k == N - 1 ? 1 : 0);
-        const int nb = neighbor[27 * s + (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)];
-        if (nb < 0) continue;
-        f[(size_t)s * N3 + q] = f[(size_t)nb * N3 + q - (dz * E * N * N + dy * E * N + dx * E)];
+        const int nb = nbs[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)];
+        const int from = q - (dz * E * N * N + dy * E * N + dx * E);  // an interior point
+        v[u] = f[(size_t)(nb < 0 ? s : nb) * N3 + from];
+        to[u] = nb < 0 ? -1 : q;
     }
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+        if (to[u] >= 0 && (int)threadIdx.x + u * kThreads < RING) blk[to[u]] = v[u];
 }
 
 // c += (6 t - sum of the 6 neighbours) inv + om2 t on interior points; one

@@ -122,6 +122,41 @@ struct ParentPass
 inline unsigned xcd_grid(long items) { return (unsigned)((items + 7) / 8 * 8); }
 __device__ inline int xcd_item(unsigned b, unsigned grid) { return (int)((b & 7) * (grid >> 3) + (b >> 3)); }
 
+// store(q, load(q)) for the COUNT points q of a block, a workgroup of T
+// threads: eight loads in flight a thread before the first of their stores
+// (a load cannot pass a store that may alias it, and one load at a time leaves
+// the launch waiting for memory: 403 blocks of 16^3, dst += a src, 12.3 -> 8.3
+// us a launch; copies of 690 us in a pass of four trees of 18^3 -> 537 us).
+template<int COUNT, int T, class Load, class Store>
+__device__ __attribute__((always_inline)) inline void each_point(Load load, Store store)
+{
+    constexpr int U = 8, R = COUNT / T;  // R whole rounds
+    using V = decltype(load(0));
+    int r = 0;
+#pragma unroll 1
+    for (; r + U <= R; r += U)
+    {
+        V v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = load((r + u) * T + (int)threadIdx.x);
+#pragma unroll
+        for (int u = 0; u < U; ++u) store((r + u) * T + (int)threadIdx.x, v[u]);
+    }
+    if constexpr (R % U != 0)
+    {
+        V v[R % U];
+#pragma unroll
+        for (int u = 0; u < R % U; ++u) v[u] = load((r + u) * T + (int)threadIdx.x);
+#pragma unroll
+        for (int u = 0; u < R % U; ++u) store((r + u) * T + (int)threadIdx.x, v[u]);
+    }
+    if constexpr (COUNT % T != 0)
+    {
+        const int q = R * T + (int)threadIdx.x;
+        if (q < COUNT) store(q, load(q));
+    }
+}
+
 namespace launch {
 
 bool supported_n(int n);
