@@ -593,7 +593,7 @@ int iblgf_gpu_clean_boundary(iblgf_gpu_ctx* ctx, int field, int level, int kind,
         ctx->solver->field_ptr(field);
         if (kind == 0) ctx->solver->clean_leaf_correction_boundary(field, level, leaf_only != 0, width);
         else
-            ctx->solver->clean_ib_region_boundary(field, level, width);
+            ctx->solver->clean_ib_region_boundary(&field, 1, level, width);
     });
 }
 

@@ -348,8 +348,7 @@ void GpuSolver::upload_forest(const std::vector<const Octree*>& trees)
     corr_level_.clear();
     smooth_lists_.clear();
     noncorr_lists_.clear();
-    p_nonleaf_all_ = DevArray<int>{};
-    p_leaf_ring_ = DevArray<int>{};
+    p_clean_ = DevArray<int>{};
     d_ramp_ = DevArray<double>{};
     step_ready_ = false;
     ghat_lap_.clear();
@@ -1771,7 +1770,10 @@ void GpuSolver::block_op(int op, const int* src, const int* dst, int level, doub
     if (op == OP_LAPLACE) fac = 1.0 / (dx * dx);
     if (op == OP_CURL_TRANSPOSE) fac = 1.0 / dx * scale;
     IBLGF_HIP(hipSetDevice(device_));
-    launch::block_op(stream_, n_, op, s, d, p_level_slots_[level].p, p_level_slots_[level].size(), fac);
+    launch::LevelFac lf;
+    lf.n = 1;
+    lf.fac[0] = fac;
+    launch::block_op(stream_, n_, op, s, d, p_level_slots_[level].p, p_level_slots_[level].size(), lf);
     IBLGF_HIP(hipGetLastError());
 }
 
@@ -1780,9 +1782,25 @@ void GpuSolver::buffer_exchange(int f, int level)
     launch::buffer_exchange(stream_, n_, F(f), p_level_slots_[level].p, p_level_slots_[level].size(), d_neighbor_.p);
 }
 
+Batch GpuSolver::table(const int* f, int k)
+{
+    if (k < 1 || k > Batch::kTab) throw std::invalid_argument("component count out of range");
+    Batch b;
+    b.k = b.ntab = k;
+    for (int c = 0; c < k; ++c) b.tab[c] = F(f[c]) - F(f[0]);
+    return b;
+}
+
+void GpuSolver::buffer_exchange(const int* f, int k, int l0, int l1)
+{
+    for (int c = 0; c < k; c += Batch::kTab)
+        launch::buffer_exchange(stream_, n_, F(f[c]), p_all_.p + lvl_begin_[l0], lvl_begin_[l1] - lvl_begin_[l0],
+            d_neighbor_.p, table(f + c, std::min(k - c, Batch::kTab)));
+}
+
 void GpuSolver::level_divergence(const int src[3], int dst, int level)
 {
-    for (int c = 0; c < 3; ++c) buffer_exchange(src[c], level);
+    buffer_exchange(src, 3, level, level + 1);
     block_op(OP_DIVERGENCE, src, &dst, level, 1.0);
     clean_leaf_correction_boundary(dst, level, true, 2);
 }
@@ -1790,7 +1808,7 @@ void GpuSolver::level_divergence(const int src[3], int dst, int level)
 void GpuSolver::level_gradient(int src, const int dst[3], int level)
 {
     block_op(OP_GRADIENT, &src, dst, level, 1.0);
-    for (int c = 0; c < 3; ++c) buffer_exchange(dst[c], level);
+    buffer_exchange(dst, 3, level, level + 1);
 }
 
 // kind 0: leaf/correction boundary (neighbour missing, or a correction block
@@ -1851,17 +1869,38 @@ const DevArray<int>& GpuSolver::corr_list(int level)
     return it->second;
 }
 
-void GpuSolver::clean_ib_region_boundary(int f, int level, int width)
+void GpuSolver::clean_ib_region_boundary(const int* f, int k, int level, int width)
 {
     const auto& l = face_clean_list(1, level, false);
-    launch::clean_faces(stream_, n_, F(f), l.p, l.size() / 2, width);
+    launch::clean_faces(stream_, n_, F(f[0]), l.p, l.size() / 2, width, table(f, k));
 }
 
-void GpuSolver::domain_clean(int f) { fill_zero(F(f)); }
-
-void GpuSolver::add(int from, int to, double scale)
+void GpuSolver::combine(const std::vector<FieldOp>& ops)
 {
-    launch::axpy_blocks(stream_, n_, F(to), F(from), p_all_.p, nb_, scale);
+    launch::CombineTable t{};
+    int                  k = 0;
+    for (const FieldOp& o : ops)
+    {
+        launch::Combine& c = t.c[k++];
+        if (o.terms.size() > 3) throw std::logic_error("field operation: too many terms");
+        c.dst = F(o.dst);
+        c.nsrc = static_cast<int>(o.terms.size());
+        for (int i = 0; i < c.nsrc; ++i)
+        {
+            c.src[i] = F(o.terms[i].f);
+            c.a[i] = o.terms[i].a;
+        }
+        c.from_zero = o.from_zero;
+        c.has_add = o.has_add;
+        c.post = o.post;
+        c.add = o.add;
+        if (k == launch::kMaxCombine)
+        {
+            launch::combine(stream_, n_, t, k, nb_);
+            k = 0;
+        }
+    }
+    launch::combine(stream_, n_, t, k, nb_);
 }
 
 SolveCounts GpuSolver::lgf_counts() const

@@ -267,28 +267,43 @@ class GpuSolver
     // ops.hpp; scale multiplies 1/dx for the curl transpose).
     void block_op(int op, const int* src, const int* dst, int level, double scale);
     void buffer_exchange(int f, int level);
+    // The same for k fields at levels [l0, l1), one launch per Batch::kTab fields.
+    void buffer_exchange(const int* f, int k, int l0, int l1);
     // Operator::levelDivergence / levelGradient (operators.hpp:522-538, 588-604)
     void level_divergence(const int src[3], int dst, int level);
     void level_gradient(int src, const int dst[3], int level);
     // Operator::clean_leaf_correction_boundary (operators.hpp:329-513) and
     // clean_ib_region_boundary (73-187)
     void clean_leaf_correction_boundary(int f, int level, bool leaf_only, int width);
-    void clean_ib_region_boundary(int f, int level, int width);
-    // Operator::domainClean (42-68) and Operator::add (3136-3153)
-    void domain_clean(int f);
-    void add(int from, int to, double scale);
+    void clean_ib_region_boundary(const int* f, int k, int level, int width);
+    // Elementwise operations over every block, in as few launches as they
+    // fit: Operator::domainClean (operators.hpp:42-68), Operator::add
+    // (3136-3153), Ifherk's copy with a scale (ifherk.hpp:1944-1960) and
+    // add_field_expression with a constant (operators.hpp:2985-3002), and
+    // chains of them rounded step by step.  No destination may be another
+    // operation's source.
+    struct FieldOp
+    {
+        struct Term
+        {
+            int    f;
+            double a;
+        };
+        int               dst;
+        std::vector<Term> terms;            // dst = sum of a f, at most three; none: zero
+        bool              from_zero = false;  // the sum starts from zero, not from the first term
+        double            post = 1.0;       // times post
+        bool              has_add = false;
+        double            add = 0.0;        // plus add
+    };
+    void combine(const std::vector<FieldOp>& ops);
     // Field operations of the IF-HERK integrator (Ifherk, ifherk.hpp) over
-    // every block: to = from * scale (copy, 1944-1960), f = f + v on every
-    // node (add_field_expression with a constant, operators.hpp:2985-3002),
-    // clean<F>(true) (1306-1350: the one-point ring of the leaves and every
-    // non-leaf block zeroed), the ramped boundary clean of
+    // every block: clean<F>(true) (1306-1350: the one-point ring of the leaves
+    // and every non-leaf block zeroed), the ramped boundary clean of
     // Ifherk::clean_leaf_correction_boundary (1352-1412), up_and_down
     // (991-1013: clean, coarsen, interpolate into the correction blocks) of k
     // components of mesh type `mesh` (component c is field index c % 3), and
     // Operator::nonlinear on one level (operators.hpp:2455-2500).
-    void copy_scaled(int from, int to, double scale);
-    void add_constant(int f, double v);
-    void clean_nonleaf(int f);
     void smooth_boundary(int f, int level, bool leaf_only);
     // Operator::maxnorm and blockRootMeanSquare of the k <= 3 component field
     // f[0..k) on every block with data, in slot order (either output may be null).
@@ -479,14 +494,20 @@ class GpuSolver
     void                 step_nonlinear(const int src[3], const int dst[3], double scale, const double frame[3]);
     void                 step_lin_sys(double alpha, int stage, bool write_prev);
     const DevArray<int>& corr_list(int level);
-    const DevArray<int>& smooth_list(bool leaf_only);
+    // The base level's ramps; kSmoothStep: the ramps with leaf_only and the
+    // correction blocks of every level, zeroed.
+    enum { kSmoothAll = 0, kSmoothLeaf = 1, kSmoothStep = 2 };
+    const DevArray<int>& smooth_list(int kind);
+    void                 smooth(const int* f, int k, int kind);
+    void                 copy3(const int from[3], const int to[3]);
+    Batch                table(const int* f, int k);  // fields f[0..k), k <= Batch::kTab
+    void                 level_op(int op, const int* src, const int* dst);  // block_op at levels >= base
     void                 step_lists();
     bool                 step_ready_ = false;
     StepFields           sf_{};
-    DevArray<int>        p_nonleaf_all_;  // non-leaf blocks at every level
-    DevArray<int>        p_leaf_ring_;    // {leaf slot, all six sides}
+    DevArray<int>        p_clean_;        // {leaf slot, all six sides}, {other slot, whole block}
     DevArray<double>     d_ramp_;         // smooth2zero ramp [2][n]
-    std::map<int, DevArray<int>> smooth_lists_;  // {base-level slot, 27-bit mask}
+    std::map<int, DevArray<int>> smooth_lists_;  // {slot, 27-bit mask, bit 27: zeroed}
 };
 
 }  // namespace iblgf_amd

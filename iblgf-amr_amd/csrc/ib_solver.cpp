@@ -47,7 +47,7 @@ IbSystem::IbSystem(GpuSolver& solver, const IbGeometry& g) : s_(solver)
 
 void IbSystem::smear(const double* d_force, const int fields[3])
 {
-    for (int c = 0; c < 3; ++c) s_.domain_clean(fields[c]);
+    s_.combine({{fields[0], {}}, {fields[1], {}}, {fields[2], {}}});
     double* f[3] = {s_.field_ptr(fields[0]), s_.field_ptr(fields[1]), s_.field_ptr(fields[2])};
     launch::ib_spread(s_.stream(), d_force, d_sp_ptr_.p, d_sp_dst_.p, d_sp_col_.p, d_sp_w_.p,
         static_cast<int>(st_.spread_ptr.size()) - 1, f);
@@ -126,7 +126,7 @@ void IbSystem::force_solve(const int fields[3], double alpha, int stage, bool wr
         launch::axpby(st, static_cast<long>(n3), -1.0, d_bcpts_.p + (stage - 1) * n3, 1.0, d_uc_.p, nullptr);
     else
         launch::force_shift(st, d_uc_.p, npoints_, bc_ + 3 * (stage - 1));
-    for (int c = 0; c < 3; ++c) s_.domain_clean(fields[c]);
+    s_.combine({{fields[0], {}}, {fields[1], {}}, {fields[2], {}}});
     stage_stats_[stage - 1] = cg(d_uc_.p, d_force_.p, alpha, step_tol_, step_maxit_);
     if (write_prev)
         IBLGF_HIP_IB(hipMemcpyAsync(prev, d_force_.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, st));
@@ -144,19 +144,17 @@ void IbSystem::project(const int fields[3], double* d_force)
 void IbSystem::apply(const double* d_fin, double* d_fout, double alpha)
 {
     const int L = s_.tree().depth - 1;
-    for (int c = 0; c < 3; ++c)
-    {
-        s_.domain_clean(field_[c]);
-        s_.domain_clean(aux_[c]);
-    }
+    s_.combine({{aux_[0], {}}, {aux_[1], {}}, {aux_[2], {}}});  // smear clears the others
     smear(d_fin, field_);
     if (std::fabs(alpha) > 1e-14) s_.apply_if_masked_batch(field_, field_, 3, alpha, MASK_IB2xIB);
     s_.level_divergence(field_, cell_, L);
-    s_.clean_ib_region_boundary(cell_, L, 2);
+    s_.clean_ib_region_boundary(&cell_, 1, L, 2);
     s_.apply_lgf_masked(cell_, cell_, MASK_xIB2IB);
     s_.level_gradient(cell_, aux_, L);
-    for (int c = 0; c < 3; ++c) s_.clean_ib_region_boundary(aux_[c], L, 2);
-    for (int c = 0; c < 3; ++c) s_.add(aux_[c], field_[c], -1.0);
+    s_.clean_ib_region_boundary(aux_, 3, L, 2);
+    std::vector<GpuSolver::FieldOp> sub;
+    for (int c = 0; c < 3; ++c) sub.push_back({field_[c], {{field_[c], 1.0}, {aux_[c], -1.0}}});
+    s_.combine(sub);
     project(field_, d_fout);
 }
 

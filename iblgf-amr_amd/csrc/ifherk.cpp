@@ -12,6 +12,7 @@
 #include "kernels.hpp"
 #include "ops.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
@@ -41,27 +42,27 @@ constexpr double kA[6] = {1.0 / 3, -1.0, 2.0, 0.0, 0.75, 0.25};
 constexpr double kC[4] = {0.0, 1.0 / 3, 1.0, 1.0};
 constexpr double coeff_a(int i, int j) { return kA[i * (i - 1) / 2 + j - 1]; }
 
-}  // namespace
-
-void GpuSolver::copy_scaled(int from, int to, double scale)
+// body(f + c, m, c) for runs of at most Batch::kTab fields, none twice in a
+// run (a field given twice is operated on twice, one after the other).
+template<class Body>
+void for_distinct(const int* f, int k, Body body)
 {
-    launch::scale_copy(stream_, n_, F(to), F(from), p_all_.p, nb_, scale);
+    for (int c = 0, m; c < k; c += m)
+    {
+        for (m = 1; c + m < k && m < Batch::kTab; ++m)
+            if (std::find(f + c, f + c + m, f[c + m]) != f + c + m) break;
+        body(f + c, m, c);
+    }
 }
 
-void GpuSolver::add_constant(int f, double v) { launch::add_const(stream_, n_, F(f), p_all_.p, nb_, v); }
+}  // namespace
 
 void GpuSolver::step_lists()
 {
-    if (p_leaf_ring_.p) return;
-    std::vector<int> nonleaf, ring;
-    for (int s = 0; s < nb_; ++s)
-    {
-        if (flags_[s] & 1u) ring.insert(ring.end(), {s, 63});
-        else
-            nonleaf.push_back(s);
-    }
-    p_nonleaf_all_.upload(nonleaf);
-    p_leaf_ring_.upload(ring);
+    if (p_clean_.p) return;
+    std::vector<int> ent;
+    for (int s = 0; s < nb_; ++s) ent.insert(ent.end(), {s, flags_[s] & 1u ? 63 : 64});
+    p_clean_.upload(ent);
     std::vector<double> r(2 * n_);
     for (int i = 0; i < n_; ++i)
     {
@@ -72,17 +73,9 @@ void GpuSolver::step_lists()
     d_ramp_.upload(r);
 }
 
-void GpuSolver::clean_nonleaf(int f)
+const DevArray<int>& GpuSolver::smooth_list(int kind)
 {
-    step_lists();
-    launch::zero_blocks(stream_, n_, F(f), p_nonleaf_all_.p, p_nonleaf_all_.size());
-    launch::clean_faces(stream_, n_, F(f), p_leaf_ring_.p, p_leaf_ring_.size() / 2, 1);
-}
-
-const DevArray<int>& GpuSolver::smooth_list(bool leaf_only)
-{
-    const int key = leaf_only ? 1 : 0;
-    auto      it = smooth_lists_.find(key);
+    auto it = smooth_lists_.find(kind);
     if (it != smooth_lists_.end()) return it->second;
     std::vector<int> ent;
     for (int s = lvl_begin_[base_level_]; s < lvl_begin_[base_level_ + 1]; ++s)
@@ -91,13 +84,44 @@ const DevArray<int>& GpuSolver::smooth_list(bool leaf_only)
         for (int i = 0; i < 27; ++i)
         {
             const int nb = neighbor_[27 * s + i];
-            if (nb < 0 || (leaf_only && (flags_[nb] & 2u))) mask |= 1 << i;
+            if (nb < 0 || (kind != kSmoothAll && (flags_[nb] & 2u))) mask |= 1 << i;
         }
-        if (mask) ent.insert(ent.end(), {s, mask});
+        if (mask && !(kind == kSmoothStep && (flags_[s] & 2u))) ent.insert(ent.end(), {s, mask});
     }
+    if (kind == kSmoothStep)
+        for (int s = lvl_begin_[base_level_]; s < nb_; ++s)
+            if (flags_[s] & 2u) ent.insert(ent.end(), {s, 1 << 27});
     DevArray<int> a;
     a.upload(ent);
-    return smooth_lists_.emplace(key, std::move(a)).first->second;
+    return smooth_lists_.emplace(kind, std::move(a)).first->second;
+}
+
+void GpuSolver::smooth(const int* f, int k, int kind)
+{
+    step_lists();
+    const auto& l = smooth_list(kind);
+    launch::smooth_ramp(stream_, n_, F(f[0]), l.p, l.size() / 2, d_ramp_.p, table(f, k));
+}
+
+void GpuSolver::level_op(int op, const int* src, const int* dst)
+{
+    const int ncs = op == OP_GRADIENT ? 1 : 3, ncd = op == OP_DIVERGENCE ? 1 : 3;
+    const double* s[3] = {nullptr, nullptr, nullptr};
+    double*       d[3] = {nullptr, nullptr, nullptr};
+    for (int c = 0; c < ncs; ++c) s[c] = F(src[c]);
+    for (int c = 0; c < ncd; ++c) d[c] = F(dst[c]);
+    for (int l0 = base_level_; l0 < depth_; l0 += launch::LevelFac::kMax)
+    {
+        launch::LevelFac lf;
+        const int        l1 = std::min(depth_, l0 + launch::LevelFac::kMax);
+        for (int l = l0; l < l1; ++l, ++lf.n)
+        {
+            lf.begin[lf.n] = lvl_begin_[l] - lvl_begin_[l0];
+            lf.fac[lf.n] = 1.0 / (dx_base_ / std::pow(2.0, l - base_level_));
+        }
+        launch::block_op(
+            stream_, n_, op, s, d, p_all_.p + lvl_begin_[l0], lvl_begin_[l1] - lvl_begin_[l0], lf);
+    }
 }
 
 // Ifherk::clean_leaf_correction_boundary (ifherk.hpp:1352-1412) on one rank:
@@ -112,9 +136,7 @@ void GpuSolver::smooth_boundary(int f, int level, bool leaf_only)
         launch::zero_blocks(stream_, n_, F(f), c.p, c.size());
     }
     if (level != base_level_) return;
-    step_lists();
-    const auto& l = smooth_list(leaf_only);
-    launch::smooth_ramp(stream_, n_, F(f), l.p, l.size() / 2, d_ramp_.p);
+    smooth(&f, 1, leaf_only ? kSmoothLeaf : kSmoothAll);
 }
 
 // Ifherk::up (ifherk.hpp:999-1004) after clean<F>(true): every component
@@ -122,42 +144,43 @@ void GpuSolver::smooth_boundary(int f, int level, bool leaf_only)
 // transfers.
 void GpuSolver::step_up(const int* f, int k, int mesh)
 {
-    for (int c = 0; c < k; ++c) clean_nonleaf(f[c]);
-    for (int c = 0; c < k; ++c)
-    {
-        Batch b;
-        b.comp0 = c % 3;
-        double* p = F(f[c]);
+    step_lists();
+    for_distinct(f, k, [&](const int* g, int m, int) {
+        launch::clean_faces(stream_, n_, F(g[0]), p_clean_.p, p_clean_.size() / 2, 1, table(g, m));
+    });
+    for_distinct(f, k, [&](const int* g, int m, int c0) {
+        Batch b = table(g, m);
+        b.comp0 = c0 % 3;
+        double* p = F(g[0]);
         for (int ls = depth_ - 2; ls >= base_level_; --ls)
             launch::transfer_gather(stream_, n_, p, p, p_coarsify_[ls].p, p_coarsify_[ls].size() / 9,
                 m_cc_restrict_.p, true, b, false, mesh);
-    }
+    });
 }
 
 // Ifherk::down_to_correction (ifherk.hpp:1006-1013): per component, each
 // level's halo fill, then the interpolation into the correction children
 // (intrp_to_correction_buffer, poisson.hpp:1015-1060).  Components are
-// independent, so each runs its level loop on its own; but the reference's
+// independent, so a level's are one launch; but the reference's
 // halo fill in that loop (buffer_exchange<From>) fills every component, so a
 // component's buffers are filled once more, from its final values, during
-// the loops of the components after it: here one more fill of each level.
+// the loops of the components after it: here one more fill of every level
+// (a fill reads and writes one level).
 void GpuSolver::step_down(const int* f, int k, int mesh)
 {
-    for (int c = 0; c < k; ++c)
-    {
-        Batch b;
-        b.comp0 = c % 3;
-        double* p = F(f[c]);
+    for_distinct(f, k, [&](const int* g, int m, int c0) {
+        Batch b = table(g, m);
+        b.comp0 = c0 % 3;
+        double* p = F(g[0]);
         for (int l = depth_ - 2; l >= base_level_; --l)
         {
-            launch::buffer_exchange(stream_, n_, p, p_level_slots_[l].p, p_level_slots_[l].size(), d_neighbor_.p);
+            buffer_exchange(g, m, l, l + 1);
             launch::transfer_scatter(stream_, n_, p, p, p_ccint_corr_[l].p, p_ccint_corr_[l].size() / 3,
                 m_cc_interp_.p, false, b, mesh);
         }
-        if (c + 1 < k)
-            for (int l = depth_ - 2; l >= base_level_; --l)
-                launch::buffer_exchange(stream_, n_, p, p_level_slots_[l].p, p_level_slots_[l].size(), d_neighbor_.p);
-    }
+        const int more = std::min(m, k - 1 - c0);
+        if (more > 0 && depth_ - 1 > base_level_) buffer_exchange(g, more, base_level_, depth_ - 1);
+    });
 }
 
 // Ifherk::up_and_down (ifherk.hpp:991-997)
@@ -190,19 +213,20 @@ void GpuSolver::step_pad_velocity(const int u[3])
 {
     const StepFields& h = sf_;
     step_up(u, 3, kMeshFace);
-    for (int c = 0; c < 3; ++c)
-    {
-        domain_clean(h.ea[c]);
-        domain_clean(h.sf[c]);
-    }
+    std::vector<FieldOp> ops;
+    for (int c = 0; c < 3; ++c) ops.insert(ops.end(), {{h.ea[c], {}}, {h.sf[c], {}}});
+    combine(ops);
+    buffer_exchange(u, 3, base_level_, depth_);
     for (int l = base_level_; l < depth_; ++l)
     {
-        for (int c = 0; c < 3; ++c) buffer_exchange(u[c], l);
         const double  dx = dx_base_ / std::pow(2.0, l - base_level_);
         const double* sp[3] = {F(u[0]), F(u[1]), F(u[2])};
         double*       dp[3] = {F(h.ea[0]), F(h.ea[1]), F(h.ea[2])};
         const auto&   list = noncorr_list(l);
-        launch::block_op(stream_, n_, OP_CURL, sp, dp, list.p, list.size(), 1.0 / dx);
+        launch::LevelFac lf;
+        lf.n = 1;
+        lf.fac[0] = 1.0 / dx;
+        launch::block_op(stream_, n_, OP_CURL, sp, dp, list.p, list.size(), lf);
     }
     for (int c = 0; c < 3; ++c) smooth_boundary(h.ea[c], base_level_, true);
     for (int c = 0; c < 3; ++c) masked_body(h.ea[c], h.sf[c], MASK_STREAM);
@@ -216,35 +240,26 @@ void GpuSolver::step_adapt_corr(const int u[3])
 {
     const StepFields& h = sf_;
     up_and_down(u, 3, kMeshFace);
-    for (int c = 0; c < 3; ++c) copy_scaled(u[c], h.q[c], 1.0);
-    for (int c = 0; c < 3; ++c)
-    {
-        domain_clean(h.g[c]);
-        domain_clean(h.fa[c]);
-    }
-    domain_clean(h.di);
-    domain_clean(h.ca);
-    for (int c = 0; c < 3; ++c) copy_scaled(h.q[c], h.r[c], 1.0);
+    copy3(u, h.q);
+    copy3(h.q, h.r);
     step_lin_sys(0.0, 1, false);
-    for (int c = 0; c < 3; ++c) domain_clean(h.r[c]);
-    domain_clean(h.di);
-    domain_clean(h.ca);
-    for (int c = 0; c < 3; ++c) add(h.q[c], h.r[c], 1.0);
+    std::vector<FieldOp> ops;
+    for (int c = 0; c < 3; ++c) ops.push_back({h.r[c], {{h.q[c], 1.0}}, true});
+    combine(ops);
     up_and_down(h.ui, 3, kMeshFace);
     step_lin_sys(0.0, 2, false);
-    domain_clean(h.di);
-    domain_clean(h.ca);
-    for (int c = 0; c < 3; ++c)
-    {
-        domain_clean(h.w2[c]);
-        copy_scaled(h.q[c], h.r[c], 1.0);
-    }
+    copy3(h.q, h.r);
     mesh_ = kMeshFace;
     if_batch_body(h.r, h.r, 3, 0.0);
     mesh_ = kMeshCell;
     up_and_down(h.ui, 3, kMeshFace);
     step_lin_sys(0.0, 3, false);
-    for (int c = 0; c < 3; ++c) copy_scaled(h.ui[c], u[c], 1.0);
+    copy3(h.ui, u);
+}
+
+void GpuSolver::copy3(const int from[3], const int to[3])
+{
+    combine({{to[0], {{from[0], 1.0}}}, {to[1], {{from[1], 1.0}}}, {to[2], {{from[2], 1.0}}}});
 }
 
 void GpuSolver::nonlinear(const int u[3], const int w[3], const int d[3], int level, double scale)
@@ -260,28 +275,19 @@ void GpuSolver::nonlinear(const int u[3], const int w[3], const int d[3], int le
 void GpuSolver::step_nonlinear(const int src[3], const int dst[3], double scale, const double frame[3])
 {
     const StepFields& h = sf_;
+    buffer_exchange(src, 3, base_level_, depth_);
+    std::vector<FieldOp> ops;
     for (int c = 0; c < 3; ++c)
-    {
-        domain_clean(h.ea[c]);
-        domain_clean(dst[c]);
-        domain_clean(h.fa[c]);
-    }
-    for (int l = base_level_; l < depth_; ++l)
-    {
-        for (int c = 0; c < 3; ++c) buffer_exchange(src[c], l);
-        block_op(OP_CURL, src, h.ea, l, 1.0);
-    }
-    for (int c = 0; c < 3; ++c)
-    {
-        copy_scaled(src[c], h.fa[c], 1.0);
-        add_constant(h.fa[c], frame[c] * -1.0);
-    }
-    for (int l = base_level_; l < depth_; ++l)
-    {
-        for (int c = 0; c < 3; ++c) buffer_exchange(h.ea[c], l);
-        for (int c = 0; c < 3; ++c) smooth_boundary(h.ea[c], l, false);
-        nonlinear(h.fa, h.ea, dst, l, scale);
-    }
+        ops.insert(ops.end(),
+            {{h.ea[c], {}}, {dst[c], {}}, {h.fa[c], {{src[c], 1.0}}, false, 1.0, true, frame[c] * -1.0}});
+    combine(ops);
+    level_op(OP_CURL, src, h.ea);
+    buffer_exchange(h.ea, 3, base_level_, depth_);
+    smooth(h.ea, 3, kSmoothAll);
+    const double* up[3] = {F(h.fa[0]), F(h.fa[1]), F(h.fa[2])};
+    const double* wp[3] = {F(h.ea[0]), F(h.ea[1]), F(h.ea[2])};
+    double*       dp[3] = {F(dst[0]), F(dst[1]), F(dst[2])};
+    launch::nonlinear(stream_, n_, up, wp, dp, p_all_.p + lvl_begin_[base_level_], nb_ - lvl_begin_[base_level_], scale);
 }
 
 // lin_sys_with_ib_solve (ifherk.hpp:1451-1517): divergence (1738-1764),
@@ -294,45 +300,34 @@ void GpuSolver::step_lin_sys(double alpha, int stage, bool write_prev)
 {
     const StepFields& h = sf_;
     up_and_down(h.r, 3, kMeshFace);
-    for (int l = base_level_; l < depth_; ++l)
-    {
-        for (int c = 0; c < 3; ++c) buffer_exchange(h.r[c], l);
-        block_op(OP_DIVERGENCE, h.r, &h.ca, l, 1.0);
-        smooth_boundary(h.ca, l, true);
-    }
+    buffer_exchange(h.r, 3, base_level_, depth_);
+    combine({{h.di, {}}, {h.ca, {}}, {h.fa[0], {}}, {h.fa[1], {}}, {h.fa[2], {}}});
+    level_op(OP_DIVERGENCE, h.r, &h.ca);
+    smooth(&h.ca, 1, kSmoothStep);
     mesh_ = kMeshCell;
     lgf_batch_body(&h.ca, &h.di, 1);
-    for (int c = 0; c < 3; ++c) domain_clean(h.fa[c]);
-    for (int l = base_level_; l < depth_; ++l)
-    {
-        block_op(OP_GRADIENT, &h.di, h.fa, l, 1.0);
-        for (int c = 0; c < 3; ++c) buffer_exchange(h.fa[c], l);
-    }
+    level_op(OP_GRADIENT, &h.di, h.fa);
+    buffer_exchange(h.fa, 3, base_level_, depth_);
     if (step_ib_)
     {
-        for (int c = 0; c < 3; ++c)
-        {
-            copy_scaled(h.r[c], h.fa2[c], 1.0);
-            add(h.fa[c], h.fa2[c], -1.0);
-        }
+        std::vector<FieldOp> diff;
+        for (int c = 0; c < 3; ++c) diff.push_back({h.fa2[c], {{h.r[c], 1.0}, {h.fa[c], -1.0}}});
+        combine(diff);
         if (std::fabs(alpha) > 1e-14) apply_if_masked_batch(h.fa2, h.fa2, 3, alpha, MASK_IB2xIB);
         step_ib_->force_solve(h.fa2, alpha, stage, write_prev);
         // pressure_correction<d_i>
-        for (int c = 0; c < 3; ++c) domain_clean(h.fa2[c]);
-        domain_clean(h.ca2);
+        combine({{h.fa2[0], {}}, {h.fa2[1], {}}, {h.fa2[2], {}}, {h.ca2, {}}});
         step_ib_->smear_add(h.fa2);
         level_divergence(h.fa2, h.ca2, depth_ - 1);
         apply_lgf_ib2amr(h.ca2, h.ca2);
-        add(h.ca2, h.di, -1.0);
-        for (int c = 0; c < 3; ++c) domain_clean(h.fa[c]);
-        for (int l = base_level_; l < depth_; ++l)
-        {
-            block_op(OP_GRADIENT, &h.di, h.fa, l, 1.0);
-            for (int c = 0; c < 3; ++c) buffer_exchange(h.fa[c], l);
-        }
+        combine({{h.di, {{h.di, 1.0}, {h.ca2, -1.0}}}, {h.fa[0], {}}, {h.fa[1], {}}, {h.fa[2], {}}});
+        level_op(OP_GRADIENT, &h.di, h.fa);
+        buffer_exchange(h.fa, 3, base_level_, depth_);
         step_ib_->smear_add(h.fa);
     }
-    for (int c = 0; c < 3; ++c) add(h.fa[c], h.r[c], -1.0);
+    std::vector<FieldOp> ops;
+    for (int c = 0; c < 3; ++c) ops.push_back({h.r[c], {{h.r[c], 1.0}, {h.fa[c], -1.0}}});
+    combine(ops);
     if (std::fabs(alpha) > 1e-14)
     {
         mesh_ = kMeshFace;
@@ -340,7 +335,7 @@ void GpuSolver::step_lin_sys(double alpha, int stage, bool write_prev)
         mesh_ = kMeshCell;
     }
     else
-        for (int c = 0; c < 3; ++c) copy_scaled(h.r[c], h.ui[c], 1.0);
+        copy3(h.r, h.ui);
 }
 
 void GpuSolver::step_prepare(const double alpha[3], int refresh)
@@ -369,8 +364,7 @@ void GpuSolver::step_prepare(const double alpha[3], int refresh)
     }
     reserve_components(6);
     step_lists();
-    smooth_list(false);
-    smooth_list(true);
+    for (int kind : {kSmoothAll, kSmoothLeaf, kSmoothStep}) smooth_list(kind);
     for (int l = 0; l < depth_; ++l)
     {
         corr_list(l);
@@ -403,33 +397,20 @@ void GpuSolver::step_body(const int u[3], int p, double dt, const double alpha[3
     }
     else
         up_and_down(u, 3, kMeshFace);
-    for (int c = 0; c < 3; ++c) copy_scaled(u[c], h.q[c], 1.0);
+    copy3(u, h.q);
+    std::vector<FieldOp> ops;
 
     // Stage 1
-    for (int c = 0; c < 3; ++c)
-    {
-        domain_clean(h.g[c]);
-        domain_clean(h.fa[c]);
-    }
-    domain_clean(h.di);
-    domain_clean(h.ca);
     step_nonlinear(u, h.g, coeff_a(1, 1) * (-dt), frame);
-    for (int c = 0; c < 3; ++c)
-    {
-        copy_scaled(h.q[c], h.r[c], 1.0);
-        add(h.g[c], h.r[c], 1.0);
-    }
+    for (int c = 0; c < 3; ++c) ops.push_back({h.r[c], {{h.q[c], 1.0}, {h.g[c], 1.0}}});
+    combine(ops);
     step_lin_sys(alpha[0], 1, true);
 
     // Stage 2
-    for (int c = 0; c < 3; ++c) domain_clean(h.r[c]);
-    domain_clean(h.di);
-    domain_clean(h.ca);
+    ops.clear();
     for (int c = 0; c < 3; ++c)
-    {
-        add(h.g[c], h.fa[c], -1.0);
-        copy_scaled(h.fa[c], h.w1[c], -1.0 / dt / coeff_a(1, 1));
-    }
+        ops.push_back({h.w1[c], {{h.fa[c], 1.0}, {h.g[c], -1.0}}, false, -1.0 / dt / coeff_a(1, 1)});
+    combine(ops);
     {
         // apply_lgf_IF<q_i, q_i> and apply_lgf_IF<w_1, w_1> at one alpha: one
         // batch of six face components, each solved in place
@@ -438,38 +419,38 @@ void GpuSolver::step_body(const int u[3], int p, double dt, const double alpha[3
         if_batch_body(qw, qw, 6, alpha[0]);
         mesh_ = kMeshCell;
     }
-    for (int c = 0; c < 3; ++c)
-    {
-        add(h.q[c], h.r[c], 1.0);
-        add(h.w1[c], h.r[c], dt * coeff_a(2, 1));
-    }
     up_and_down(h.ui, 3, kMeshFace);
     step_nonlinear(h.ui, h.g, coeff_a(2, 2) * (-dt), frame + 3);
-    for (int c = 0; c < 3; ++c) add(h.g[c], h.r[c], 1.0);
+    ops.clear();
+    for (int c = 0; c < 3; ++c)
+        ops.push_back({h.r[c], {{h.q[c], 1.0}, {h.w1[c], dt * coeff_a(2, 1)}, {h.g[c], 1.0}}, true});
+    combine(ops);
     step_lin_sys(alpha[1], 2, true);
 
     // Stage 3
-    domain_clean(h.di);
-    domain_clean(h.ca);
-    for (int c = 0; c < 3; ++c) domain_clean(h.w2[c]);
+    ops.clear();
     for (int c = 0; c < 3; ++c)
-    {
-        add(h.g[c], h.fa[c], -1.0);
-        copy_scaled(h.fa[c], h.w2[c], -1.0 / dt / coeff_a(2, 2));
-        copy_scaled(h.q[c], h.r[c], 1.0);
-        add(h.w1[c], h.r[c], dt * coeff_a(3, 1));
-        add(h.w2[c], h.r[c], dt * coeff_a(3, 2));
-    }
+        ops.push_back({h.w2[c], {{h.fa[c], 1.0}, {h.g[c], -1.0}}, false, -1.0 / dt / coeff_a(2, 2)});
+    combine(ops);
+    ops.clear();
+    for (int c = 0; c < 3; ++c)
+        ops.push_back(
+            {h.r[c], {{h.q[c], 1.0}, {h.w1[c], dt * coeff_a(3, 1)}, {h.w2[c], dt * coeff_a(3, 2)}}});
+    combine(ops);
     mesh_ = kMeshFace;
     if_batch_body(h.r, h.r, 3, alpha[1]);
     mesh_ = kMeshCell;
     up_and_down(h.ui, 3, kMeshFace);
     step_nonlinear(h.ui, h.g, coeff_a(3, 3) * (-dt), frame + 6);
-    for (int c = 0; c < 3; ++c) add(h.g[c], h.r[c], 1.0);
+    ops.clear();
+    for (int c = 0; c < 3; ++c) ops.push_back({h.r[c], {{h.r[c], 1.0}, {h.g[c], 1.0}}});
+    combine(ops);
     step_lin_sys(alpha[2], 3, true);
 
-    for (int c = 0; c < 3; ++c) copy_scaled(h.ui[c], u[c], 1.0);
-    if (p >= 0) copy_scaled(h.di, p, 1.0 / coeff_a(3, 3) / dt);
+    ops.clear();
+    for (int c = 0; c < 3; ++c) ops.push_back({u[c], {{h.ui[c], 1.0}}});
+    if (p >= 0) ops.push_back({p, {{h.di, 1.0 / coeff_a(3, 3) / dt}}});
+    combine(ops);
     IBLGF_HIP_HK(hipGetLastError());
 }
 

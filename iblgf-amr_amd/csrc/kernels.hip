@@ -51,11 +51,11 @@ __device__ inline void twiddles(double2* W, int P)
 // Elementwise block kernels
 // ---------------------------------------------------------------------------
 template<int N>
-__global__ __launch_bounds__(kThreads) void k_zero(double* f, const int* slots, int count, long cs)
+__global__ __launch_bounds__(kThreads) void k_zero(double* f, const int* slots, int count, CompOff cs)
 {
     const int b = blockIdx.x;
     if (b >= count) return;
-    double* p = f + blockIdx.y * cs + (size_t)slots[b] * Geo<N>::N3;
+    double* p = f + cs(blockIdx.y) + (size_t)slots[b] * Geo<N>::N3;
     for (int q = threadIdx.x; q < Geo<N>::N3; q += kThreads) p[q] = 0.0;
 }
 
@@ -103,19 +103,6 @@ __global__ __launch_bounds__(kThreads) void k_copy_table(
     else
         copy_block<N>(reinterpret_cast<float*>(dst.p[c]) + off, reinterpret_cast<const float*>(src.p[c]) + off,
             interior);
-}
-
-template<int N>
-__global__ __launch_bounds__(kThreads) void k_axpy(
-    double* dst, const double* src, const int* slots, int count, double a, long cs)
-{
-#pragma clang fp contract(off)  // product and sum rounded separately (Operator::add)
-    const int b = blockIdx.x;
-    if (b >= count) return;
-    const size_t off = blockIdx.y * cs + (size_t)slots[b] * Geo<N>::N3;
-    each_point<Geo<N>::N3, kThreads>([=](int q) {
-#pragma clang fp contract(off)
-        return dst[off + q] + src[off + q] * a; }, [=](int q, double v) { dst[off + q] = v; });
 }
 
 // ---------------------------------------------------------------------------
@@ -196,7 +183,7 @@ __device__ inline int side_mat(int mesh, int fi, int axis, int bit)
 template<int N, bool GATHER>
 __global__ __launch_bounds__((TransferGeo<N, GATHER>::T)) void k_transfer(const double* __restrict__ src,
     double* __restrict__ dst, const int* __restrict__ entries, int count, const double* __restrict__ mats,
-    int accumulate, int ring0, long cs, int mesh, int comp0)
+    int accumulate, int ring0, CompOff cs, int mesh, int comp0)
 {
     using G = TransferGeo<N, GATHER>;
     constexpr int     KZ = G::KZ, OG = G::OG, NN = G::NN, N3 = Geo<N>::N3, NX = GATHER ? 2 : 1;
@@ -207,8 +194,8 @@ __global__ __launch_bounds__((TransferGeo<N, GATHER>::T)) void k_transfer(const 
     const int         fi = (comp0 + (int)blockIdx.y) % 3;
     const int*        ent = entries + (GATHER ? 9 : 3) * e;
     const int         id = GATHER ? 0 : ent[2];  // sides of the one transfer
-    src += blockIdx.y * cs;
-    dst += blockIdx.y * cs + (size_t)ent[0] * N3 + k0 * NN;
+    src += cs(blockIdx.y);
+    dst += cs(blockIdx.y) + (size_t)ent[0] * N3 + k0 * NN;
     for (int it = threadIdx.x; it < NX * NX * NN; it += G::T)
     {
         const int  xy = it / NN, col = it - xy * NN, y = col / N, x = col - y * N;
@@ -312,12 +299,12 @@ __device__ inline int ring_point(int r)
 // neighbour (the reads are interior points only, so blocks run concurrently).
 template<int N>
 __global__ __launch_bounds__(kThreads) void k_buffer_exchange(
-    double* f, const int* slots, int count, const int* __restrict__ neighbor, long cs)
+    double* f, const int* slots, int count, const int* __restrict__ neighbor, CompOff cs)
 {
     constexpr int N3 = Geo<N>::N3, E = Geo<N>::E, RING = N3 - E * E * E;
     const int b = blockIdx.x;
     if (b >= count) return;
-    f += blockIdx.y * cs;
+    f += cs(blockIdx.y);
     const int s = slots[b];
     // every value of the thread loaded before the first is stored
     constexpr int R = (RING + kThreads - 1) / kThreads;
@@ -1271,7 +1258,7 @@ template<int N> struct RunZero
 {
     static void run(hipStream_t s, double* f, const int* slots, int count, const Batch& b)
     {
-        hipLaunchKernelGGL(k_zero<N>, dim3(count, b.k), dim3(kThreads), 0, s, f, slots, count, b.fstride);
+        hipLaunchKernelGGL(k_zero<N>, dim3(count, b.k), dim3(kThreads), 0, s, f, slots, count, CompOff(b));
     }
 };
 template<int N> struct RunCopy
@@ -1291,14 +1278,6 @@ template<int N> struct RunCopyTable
         hipLaunchKernelGGL(k_copy_table<N>, dim3(count, k), dim3(kThreads), 0, s, d, src, slots, count, interior);
     }
 };
-template<int N> struct RunAxpy
-{
-    static void run(hipStream_t s, double* d, const double* src, const int* slots, int count, double a,
-        const Batch& b)
-    {
-        hipLaunchKernelGGL(k_axpy<N>, dim3(count, b.k), dim3(kThreads), 0, s, d, src, slots, count, a, b.fstride);
-    }
-};
 template<int N> struct RunGather
 {
     static void run(hipStream_t s, const double* src, double* dst, const int* e, int count, const double* m,
@@ -1306,7 +1285,7 @@ template<int N> struct RunGather
     {
         using G = TransferGeo<N, true>;
         hipLaunchKernelGGL((k_transfer<N, true>), dim3(xcd_grid((long)count * G::PARTS), b.k), dim3(G::T), 0, s, src, dst,
-            e, count, m, accumulate, ring0, b.fstride, mesh, b.comp0);
+            e, count, m, accumulate, ring0, CompOff(b), mesh, b.comp0);
     }
 };
 template<int N> struct RunScatter
@@ -1316,7 +1295,7 @@ template<int N> struct RunScatter
     {
         using G = TransferGeo<N, false>;
         hipLaunchKernelGGL((k_transfer<N, false>), dim3(xcd_grid((long)count * G::PARTS), b.k), dim3(G::T), 0, s, src, dst,
-            e, count, m, acc, 0, b.fstride, mesh, b.comp0);
+            e, count, m, acc, 0, CompOff(b), mesh, b.comp0);
     }
 };
 template<int N> struct RunHalo
@@ -1324,7 +1303,7 @@ template<int N> struct RunHalo
     static void run(hipStream_t s, double* f, const int* slots, int count, const int* nb, const Batch& b)
     {
         hipLaunchKernelGGL(k_buffer_exchange<N>, dim3(count, b.k), dim3(kThreads), 0, s, f, slots, count, nb,
-            b.fstride);
+            CompOff(b));
     }
 };
 template<int N> struct RunStencil
@@ -1501,11 +1480,6 @@ void copy_blocks_table(hipStream_t s, int n, const FieldTable& dst, const FieldT
 {
     if (k < 1 || k > kMaxFieldTable) throw std::invalid_argument("copy_blocks_table: component count out of range");
     if (count > 0) dispatch_n<RunCopyTable>(n, s, dst, src, slots, count, interior_only ? 1 : 0, k);
-}
-void axpy_blocks(hipStream_t s, int n, double* dst, const double* src, const int* slots, int count, double a,
-    const Batch& b)
-{
-    if (count > 0) dispatch_n<RunAxpy>(n, s, dst, src, slots, count, a, b);
 }
 void transfer_gather(hipStream_t s, int n, const double* src, double* dst, const int* entries, int count,
     const double* mats, bool accumulate, const Batch& b, bool children_interior, int mesh)

@@ -55,6 +55,25 @@ struct Batch
     // Field index of component 0 (vector fields: component c is field index
     // (comp0 + c) % 3), for the mesh-type level transfers.
     int comp0 = 0;
+    // Fields at unrelated addresses: component c starts tab[c] doubles in for
+    // c < ntab <= kTab (ntab 0: fstride).  Taken by zero_blocks, the transfers
+    // and buffer_exchange.
+    static constexpr int kTab = 8;
+    int  ntab = 0;
+    long tab[kTab] = {};
+};
+
+// Where component c of a launch starts, as a kernel argument.
+struct CompOff
+{
+    long stride;
+    int  ntab;
+    long tab[Batch::kTab];
+    CompOff(const Batch& b) : stride(b.fstride), ntab(b.ntab)
+    {
+        for (int c = 0; c < Batch::kTab; ++c) tab[c] = b.tab[c];
+    }
+    __device__ long operator()(int c) const { return ntab ? tab[c] : c * stride; }
 };
 
 // Mesh types of the level transfers (MeshObject of the reference).
@@ -169,8 +188,6 @@ void copy_blocks(hipStream_t s, int n, double* dst, const double* src, const int
 // The same for k components whose fields sit at unrelated addresses, in one launch.
 void copy_blocks_table(hipStream_t s, int n, const FieldTable& dst, const FieldTable& src, const int* slots,
     int count, bool interior_only, int k);
-void axpy_blocks(hipStream_t s, int n, double* dst, const double* src, const int* slots, int count,
-    double a, const Batch& b = {});
 
 // dst[entry.parent] (=|+=) sum_c K(child) for entries {parent, child[8]}; K
 // built from side matrices (row = output point, col = input point):

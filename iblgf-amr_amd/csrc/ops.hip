@@ -16,8 +16,6 @@
 // each result is the reference's sequence of roundings.
 #include "ops.hpp"
 
-#include "kernels.hpp"
-
 #include <stdexcept>
 
 namespace iblgf_amd {
@@ -28,12 +26,15 @@ constexpr int kThreads = 256;
 template<int N, int OP>
 __global__ __launch_bounds__(kThreads) void k_block_op(const double* __restrict__ s0, const double* __restrict__ s1,
     const double* __restrict__ s2, double* __restrict__ d0, double* __restrict__ d1, double* __restrict__ d2,
-    const int* __restrict__ slots, int count, double fac)
+    const int* __restrict__ slots, int count, launch::LevelFac levels)
 {
 #pragma clang fp contract(off)
     constexpr int E = N - 2, NN = N * N, N3 = N * N * N, E3 = E * E * E;
     const int     b = blockIdx.x;
     if (b >= count) return;
+    double fac = levels.fac[0];
+    for (int l = 1; l < levels.n; ++l)
+        if (b >= levels.begin[l]) fac = levels.fac[l];
     const size_t off = (size_t)slots[b] * N3;
     for (int t = threadIdx.x; t < E3; t += kThreads)
     {
@@ -102,20 +103,20 @@ __global__ __launch_bounds__(kThreads) void k_block_op(const double* __restrict_
 
 template<int N>
 __global__ __launch_bounds__(kThreads) void k_clean_faces(double* f, const int* __restrict__ entries, int count,
-    int width)
+    int width, CompOff cs)
 {
     constexpr int N3 = N * N * N;
     const int     b = blockIdx.x;
     if (b >= count) return;
     const int    mask = entries[2 * b + 1];
-    double*      blk = f + (size_t)entries[2 * b] * N3;
+    double*      blk = f + cs(blockIdx.y) + (size_t)entries[2 * b] * N3;
     for (int q = threadIdx.x; q < N3; q += kThreads)
     {
         const int i = q % N, j = (q / N) % N, k = q / (N * N);
         const bool z = ((mask & 1) && k < width) || ((mask & 32) && k >= N - width);
         const bool y = ((mask & 2) && j < width) || ((mask & 16) && j >= N - width);
         const bool x = ((mask & 4) && i < width) || ((mask & 8) && i >= N - width);
-        if (x || y || z) blk[q] = 0.0;
+        if (x || y || z || (mask & 64)) blk[q] = 0.0;
     }
 }
 
@@ -353,28 +354,38 @@ __global__ __launch_bounds__(kThreads) void k_nonlinear(const double* __restrict
     }
 }
 
-// dst = src * a, every node of the listed blocks.
-template<int N>
-__global__ __launch_bounds__(kThreads) void k_scale_copy(
-    double* __restrict__ dst, const double* __restrict__ src, const int* __restrict__ slots, int count, double a)
+// Launches of a few microseconds each are bound by their count: a step's
+// elementwise operations are a table of combinations, up to twelve a launch.
+template<int N, int NSRC>
+__device__ inline void combine_block(const launch::Combine& c, size_t off)
 {
-    constexpr int N3 = N * N * N;
-    const int     b = blockIdx.x;
-    if (b >= count) return;
-    const size_t off = (size_t)slots[b] * N3;
-    each_point<N3, kThreads>([=](int t) { return src[off + t] * a; }, [=](int t, double v) { dst[off + t] = v; });
+    each_point<N * N * N, kThreads>(
+        [&](int q) {
+#pragma clang fp contract(off)
+            double v = 0.0;
+            if constexpr (NSRC > 0)
+            {
+                v = c.src[0][off + q] * c.a[0];
+                if (c.from_zero) v = 0.0 + v;
+            }
+            if constexpr (NSRC > 1) v = v + c.src[1][off + q] * c.a[1];
+            if constexpr (NSRC > 2) v = v + c.src[2][off + q] * c.a[2];
+            v = v * c.post;
+            return c.has_add ? v + c.add : v;
+        },
+        [&](int q, double v) { c.dst[off + q] = v; });
 }
 
-// f = f + v, every node of the listed blocks.
 template<int N>
-__global__ __launch_bounds__(kThreads) void k_add_const(double* __restrict__ f, const int* __restrict__ slots,
-    int count, double v)
+__global__ __launch_bounds__(kThreads) void k_combine(launch::CombineTable t)
 {
-    constexpr int N3 = N * N * N;
-    const int     b = blockIdx.x;
-    if (b >= count) return;
-    const size_t off = (size_t)slots[b] * N3;
-    each_point<N3, kThreads>([=](int t) { return f[off + t] + v; }, [=](int t, double w) { f[off + t] = w; });
+    const launch::Combine& c = t.c[blockIdx.y];
+    const size_t           off = (size_t)blockIdx.x * (N * N * N);
+    if (c.nsrc == 0) combine_block<N, 0>(c, off);
+    else if (c.nsrc == 1) combine_block<N, 1>(c, off);
+    else if (c.nsrc == 2) combine_block<N, 2>(c, off);
+    else
+        combine_block<N, 3>(c, off);
 }
 
 // Operator::smooth2zero (operators.hpp:653-760) for every neighbour i set in
@@ -386,21 +397,21 @@ __global__ __launch_bounds__(kThreads) void k_add_const(double* __restrict__ f, 
 // ramp values are six that stay in registers (31.7 -> 13.7 us a launch).
 template<int N>
 __global__ __launch_bounds__(kThreads) void k_smooth_ramp(
-    double* __restrict__ f, const int* __restrict__ entries, int count, const double* __restrict__ ramp)
+    double* __restrict__ f, const int* __restrict__ entries, int count, const double* __restrict__ ramp, CompOff cs)
 {
 #pragma clang fp contract(off)
     constexpr int N3 = N * N * N;
     const int     k = blockIdx.x % N, b = blockIdx.x / N;  // a workgroup per z plane
     if (b >= count) return;
     const int    mask = entries[2 * b + 1];
-    double*      plane = f + (size_t)entries[2 * b] * N3 + k * N * N;
+    double*      plane = f + cs(blockIdx.y) + (size_t)entries[2 * b] * N3 + k * N * N;
     const double z0 = ramp[k], z2 = ramp[N + k];
     for (int t = threadIdx.x; t < N * N; t += kThreads)
     {
         const int    i = t % N, j = t / N;
         const double x0 = ramp[i], x2 = ramp[N + i], y0 = ramp[j], y2 = ramp[N + j];
-        double       v = plane[t];
-        for (int left = mask; left; left &= left - 1)
+        double       v = (mask >> 27) & 1 ? 0.0 : plane[t];
+        for (int left = mask & ((1 << 27) - 1); left; left &= left - 1)
         {
             const int g = __builtin_ctz(left), gx = g % 3, gy = (g / 3) % 3, gz = g / 9;
             double    square = 0.0;
@@ -414,7 +425,7 @@ __global__ __launch_bounds__(kThreads) void k_smooth_ramp(
 }
 
 template<template<int> class F, typename... Args>
-void dispatch_n(int n, Args... args)
+void dispatch_n(int n, const Args&... args)
 {
     switch (n)
     {
@@ -431,7 +442,7 @@ template<int N>
 struct RunOp
 {
     static void run(hipStream_t s, int op, const double* const* src, double* const* dst, const int* slots, int count,
-        double fac)
+        const launch::LevelFac& fac)
     {
         const dim3 g(count), t(kThreads);
 #define IBLGF_OP(K)                                                                                           \
@@ -463,9 +474,10 @@ struct RunNorms
 template<int N>
 struct RunClean
 {
-    static void run(hipStream_t s, double* f, const int* entries, int count, int width)
+    static void run(hipStream_t s, double* f, const int* entries, int count, int width, const Batch& b)
     {
-        hipLaunchKernelGGL((k_clean_faces<N>), dim3(count), dim3(kThreads), 0, s, f, entries, count, width);
+        hipLaunchKernelGGL((k_clean_faces<N>), dim3(count, b.k), dim3(kThreads), 0, s, f, entries, count, width,
+            CompOff(b));
     }
 };
 
@@ -488,27 +500,20 @@ struct RunNonlinear
     }
 };
 template<int N>
-struct RunScaleCopy
+struct RunCombine
 {
-    static void run(hipStream_t s, double* dst, const double* src, const int* slots, int count, double a)
+    static void run(hipStream_t s, const launch::CombineTable& t, int k, int nblocks)
     {
-        hipLaunchKernelGGL((k_scale_copy<N>), dim3(count), dim3(kThreads), 0, s, dst, src, slots, count, a);
-    }
-};
-template<int N>
-struct RunAddConst
-{
-    static void run(hipStream_t s, double* f, const int* slots, int count, double v)
-    {
-        hipLaunchKernelGGL((k_add_const<N>), dim3(count), dim3(kThreads), 0, s, f, slots, count, v);
+        hipLaunchKernelGGL((k_combine<N>), dim3(nblocks, k), dim3(kThreads), 0, s, t);
     }
 };
 template<int N>
 struct RunSmooth
 {
-    static void run(hipStream_t s, double* f, const int* entries, int count, const double* ramp)
+    static void run(hipStream_t s, double* f, const int* entries, int count, const double* ramp, const Batch& b)
     {
-        hipLaunchKernelGGL((k_smooth_ramp<N>), dim3(count * N), dim3(kThreads), 0, s, f, entries, count, ramp);
+        hipLaunchKernelGGL((k_smooth_ramp<N>), dim3(count * N, b.k), dim3(kThreads), 0, s, f, entries, count, ramp,
+            CompOff(b));
     }
 };
 
@@ -527,23 +532,19 @@ void remap_blocks(hipStream_t s, int n, double* dst, const double* src, const in
     if (count > 0) dispatch_n<RunRemap>(n, s, dst, src, pairs, count);
 }
 
-void scale_copy(hipStream_t s, int n, double* dst, const double* src, const int* slots, int count, double a)
+void combine(hipStream_t s, int n, const CombineTable& t, int k, int nblocks)
 {
-    if (count > 0) dispatch_n<RunScaleCopy>(n, s, dst, src, slots, count, a);
+    if (k < 0 || k > kMaxCombine) throw std::invalid_argument("combine: count out of range");
+    if (k > 0 && nblocks > 0) dispatch_n<RunCombine>(n, s, t, k, nblocks);
 }
 
-void add_const(hipStream_t s, int n, double* f, const int* slots, int count, double v)
+void smooth_ramp(hipStream_t s, int n, double* f, const int* entries, int count, const double* ramp, const Batch& b)
 {
-    if (count > 0) dispatch_n<RunAddConst>(n, s, f, slots, count, v);
-}
-
-void smooth_ramp(hipStream_t s, int n, double* f, const int* entries, int count, const double* ramp)
-{
-    if (count > 0) dispatch_n<RunSmooth>(n, s, f, entries, count, ramp);
+    if (count > 0) dispatch_n<RunSmooth>(n, s, f, entries, count, ramp, b);
 }
 
 void block_op(hipStream_t s, int n, int op, const double* const src[3], double* const dst[3], const int* slots,
-    int count, double fac)
+    int count, const LevelFac& fac)
 {
     if (count > 0) dispatch_n<RunOp>(n, s, op, src, dst, slots, count, fac);
 }
@@ -554,10 +555,10 @@ void block_norms(hipStream_t s, int n, const double* const c[3], int k, const in
     if (count > 0) dispatch_n<RunNorms>(n, s, c, k, slots, count, out);
 }
 
-void clean_faces(hipStream_t s, int n, double* f, const int* entries, int count, int width)
+void clean_faces(hipStream_t s, int n, double* f, const int* entries, int count, int width, const Batch& b)
 {
     if (width < 0 || width > n) throw std::runtime_error("clean width out of range");
-    if (count > 0) dispatch_n<RunClean>(n, s, f, entries, count, width);
+    if (count > 0) dispatch_n<RunClean>(n, s, f, entries, count, width, b);
 }
 
 void ib_spread(hipStream_t s, const double* force, const int* row_ptr, const int* row_dst, const int* col,

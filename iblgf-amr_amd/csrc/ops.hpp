@@ -10,6 +10,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "kernels.hpp"
+
 namespace iblgf_amd {
 
 enum BlockOp
@@ -25,13 +27,22 @@ namespace launch {
 
 // dst = op(src) over the interior of each listed block; fac = 1/dx (1/dx^2
 // for the Laplacian, (1/dx)*scale for the curl transpose).
+// Several levels in one launch: entry b takes the fac of the last level with begin <= b.
+struct LevelFac
+{
+    static constexpr int kMax = 16;
+    int    n = 0;
+    int    begin[kMax];
+    double fac[kMax];
+};
 void block_op(hipStream_t s, int n, int op, const double* const src[3], double* const dst[3], const int* slots,
-    int count, double fac);
+    int count, const LevelFac& fac);
 
 // Zero `width` planes on the sides named by the 6-bit face mask of each
 // entry {slot, mask}; bit b is neighbour slot {4,10,12,14,16,22}[b]
-// (z-, y-, x-, x+, y+, z+).
-void clean_faces(hipStream_t s, int n, double* f, const int* entries, int count, int width);
+// (z-, y-, x-, x+, y+, z+), bit 6 the whole block.
+void clean_faces(
+    hipStream_t s, int n, double* f, const int* entries, int count, int width, const Batch& b = {});
 // Per listed block: the largest sum of squares of the k <= 3 components over
 // its interior points (out[2b]) and the total of those sums (out[2b+1]).
 void block_norms(hipStream_t s, int n, const double* const c[3], int k, const int* slots, int count, double* out);
@@ -43,12 +54,30 @@ void nonlinear(hipStream_t s, int n, const double* const u[3], const double* con
     const int* slots, int count, double scale);
 // dst[new slot] = src[old slot] for pairs {old, new}, whole blocks.
 void remap_blocks(hipStream_t s, int n, double* dst, const double* src, const int* pairs, int count);
-// dst = src * a and f = f + v on every node of the listed blocks.
-void scale_copy(hipStream_t s, int n, double* dst, const double* src, const int* slots, int count, double a);
-void add_const(hipStream_t s, int n, double* f, const int* slots, int count, double v);
+// dst = (a[0] src[0] + a[1] src[1] + a[2] src[2]) post + add over every node of
+// a field, products and sums rounded one after the other in that order (no
+// source: zero; from_zero: 0 + a[0] src[0] first; add only where has_add).
+struct Combine
+{
+    double*       dst;
+    const double* src[3];
+    double        a[3];
+    int           nsrc;
+    int           from_zero, has_add;
+    double        post, add;
+};
+constexpr int kMaxCombine = 12;
+struct CombineTable
+{
+    Combine c[kMaxCombine];
+};
+// The first k combinations in one launch; dst of one is no src of another.
+void combine(hipStream_t s, int n, const CombineTable& t, int k, int nblocks);
 // Operator::smooth2zero for entries {slot, 27-bit neighbour mask}; ramp[2][n]
-// holds the ramp at node index idx towards the low and the high side.
-void smooth_ramp(hipStream_t s, int n, double* f, const int* entries, int count, const double* ramp);
+// holds the ramp at node index idx towards the low and the high side.  Bit 27:
+// the block is zeroed instead.
+void smooth_ramp(hipStream_t s, int n, double* f, const int* entries, int count, const double* ramp,
+    const Batch& b = {});
 
 // Immersed-boundary transfer with precomputed delta weights.
 // spread: field_c[node] = sum_k force[col_k] * w_k over the rows of node,
