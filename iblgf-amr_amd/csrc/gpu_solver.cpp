@@ -729,7 +729,13 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
         std::vector<MacGroup> groups;
         std::vector<MacSrc>   srcs;
         long                  m_nfull = 0, m_pairs_full = 0, m_pop[8] = {};
-        std::vector<int>      psrc, ptgt, pbegin(1, 0), pent;  // as ParentPass
+        std::vector<int>      psrc, ptgt;  // as ParentPass
+        struct Near  // source of a target parent
+        {
+            int source, offset, target;
+        };
+        std::vector<Near> pnear;
+        std::vector<std::array<int, 4>> pcoord;  // tree and place of each target parent
         std::unordered_map<uint64_t, int> pidx;
         long                  pairs_parents = 0, entries_parents = 0;
         for (auto& b : gb)
@@ -758,9 +764,9 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
                         psrc.insert(psrc.end(), it->second.begin(), it->second.end());
                         for (int s : it->second) p.par_nfwd += s >= 0 ? 1 : 0;
                     }
-                    pent.push_back(at.first->second * 32 + o);
+                    pnear.push_back({at.first->second, o, static_cast<int>(ptgt.size() / 8) - 1});
                 }
-                pbegin.push_back(static_cast<int>(pent.size()));
+                pcoord.push_back({static_cast<int>(b.tree), b.coord[0], b.coord[1], b.coord[2]});
                 pairs_parents += gpairs;
                 entries_parents += static_cast<long>(b.ent.size());
                 continue;
@@ -808,6 +814,46 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
             p.npar_tgt = static_cast<int>(ptgt.size() / 8);
             p.par_src.upload(psrc);
             p.par_tgt.upload(ptgt);
+            // groups of targets that share sources, 2 x 2 parents in x and y; a
+            // group's entries by the source's place, z slowest, so that every
+            // target meets its own in the order of their offsets
+            std::map<std::array<int, 4>, int> gidx;
+            auto lane = [&](int t) { return (pcoord[t][1] & 1) | (pcoord[t][2] & 1) << 1; };
+            std::vector<int4>                 group;
+            std::vector<int>                  gof(pcoord.size());
+            for (int t = 0; t < p.npar_tgt; ++t)
+            {
+                const auto& c = pcoord[t];
+                const auto  at = gidx.emplace(
+                    std::array<int, 4>{c[0], c[3], c[2] >> 1, c[1] >> 1}, static_cast<int>(group.size()));
+                if (at.second) group.push_back(make_int4(-1, -1, -1, -1));
+                gof[t] = at.first->second;
+                (&group[gof[t]].x)[lane(t)] = t;
+            }
+            // {group, z, y, x, source, target of the group, offset}
+            std::vector<std::array<int, 7>> near;
+            near.reserve(pnear.size());
+            for (const Near& e : pnear)
+            {
+                const auto& c = pcoord[e.target];
+                const int   o = e.offset;
+                near.push_back({gof[e.target], c[3] + o / 9, c[2] + (o / 3) % 3, c[1] + o % 3, e.source,
+                    lane(e.target), o});
+            }
+            std::sort(near.begin(), near.end());
+            std::vector<int>  pbegin(group.size() + 1, 0);
+            std::vector<int2> pent;
+            for (size_t i = 0; i < near.size(); ++i)
+            {
+                const auto& e = near[i];
+                if (i == 0 || !std::equal(e.begin(), e.begin() + 5, near[i - 1].begin()))
+                    pent.push_back(make_int2(e[4], kParentNone * 0x01010101));
+                int& w = pent.back().y;
+                w = (w & ~(255 << 8 * e[5])) | e[6] << 8 * e[5];
+                pbegin[e[0] + 1] = static_cast<int>(pent.size());
+            }
+            for (size_t g = 0; g < group.size(); ++g) pbegin[g + 1] = std::max(pbegin[g + 1], pbegin[g]);
+            p.par_group.upload(group);
             p.par_begin.upload(pbegin);
             p.par_ent.upload(pent);
             p.par_npairs = p.par_stats.npairs = p.par_stats.pairs_full = pairs_parents;
@@ -1128,7 +1174,8 @@ void GpuSolver::run_parents(PassPlan& p, double scale, const Batch& b)
 {
     const double2* g = parent_ghat();
     reserve_parents();
-    const ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt, g,
+    const ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_group.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt,
+        static_cast<int>(p.par_group.n), g,
         par_sspec_.p, par_tspec_.p, par_mid_.p};
     launch::parent_pass(stream_, n_, precision_, pp, wp_.src, wp_.tgt, scale, b);
 }

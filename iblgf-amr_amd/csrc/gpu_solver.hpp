@@ -85,7 +85,9 @@ struct PassPlan
     // Laplace passes: the level-L sums by transforms of whole parents
     // (parent_fft.hip), the blocks that take that path, and the statistics of
     // their pairs (the entries a block-wise plan would have).
-    DevArray<int>                    par_src, par_tgt, par_begin, par_ent;
+    DevArray<int>                    par_src, par_tgt, par_begin;
+    DevArray<int4>                   par_group;
+    DevArray<int2>                   par_ent;
     int                              npar_src = 0, npar_tgt = 0;
     long                             par_nfwd = 0, par_ninv = 0, par_npairs = 0;
     MacLevelPlan                     par_stats;
@@ -104,10 +106,10 @@ struct SolveCounts
 enum KernelClass
 {
     KC_FORWARD = 0,   // forward block DFT
-    KC_MAC = 1,       // spectral multiply-accumulate
+    KC_MAC = 1,       // spectral multiply-accumulate; passes of whole parents with their transforms
     KC_INVERSE = 2,   // inverse block DFT
     KC_TRANSFER = 3,  // anterpolation / interpolation / coarsify
-    KC_OTHER = 4,     // copies, halo, correction stencil
+    KC_OTHER = 4,     // copies, halo, correction stencil, separable integrating factor
     KC_COUNT = 5
 };
 

@@ -115,18 +115,23 @@ struct ParentGeo
     int M, W, P, H, NF;
 };
 // src_child[nsrc][8], tgt_child[ntgt][8]: block slots of the children (-1:
-// not a source / target); entries begin[t] .. begin[t + 1] of target t: source
-// parent * 32 + offset (ox + 1) + 3 (oy + 1) + 9 (oz + 1) of the source.
+// not a source / target).  group[ngroup]: up to four target parents that are
+// neighbours (-1: none); entries begin[g] .. begin[g + 1] of group g: {source
+// parent, offset (ox + 1) + 3 (oy + 1) + 9 (oz + 1) of the source from target
+// t of the group in byte t (kParentNone: not a source of that target)}, every
+// target's offsets ascending.
 // ghat: 14 spectra of parent_spectra (offsets 13 to 26).  Scratch for k components: sspec and
 // tspec a spectrum per source / target parent (FP64, or FP32 with prec > 0),
 // mid H values a column for the larger of nsrc M M and ntgt W W columns.
+constexpr int kParentNone = 27;  // a row of zeros
 struct ParentPass
 {
     const int*     src_child;
     const int*     tgt_child;
+    const int4*    group;
     const int*     begin;
-    const int*     entries;
-    int            nsrc, ntgt;
+    const int2*    entries;
+    int            nsrc, ntgt, ngroup;
     const double2* ghat;
     void*          sspec;
     void*          tspec;

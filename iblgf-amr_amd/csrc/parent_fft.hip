@@ -432,42 +432,51 @@ __global__ __launch_bounds__(Par<N>::T) __attribute__((amdgpu_waves_per_eu(5))) 
 // ---------------------------------------------------------------------------
 // Spectral products: tspec[target] = sum over its entries of
 // ghat[offset] * sspec[source].  A workgroup takes 64 frequencies and a run of
-// (target, component) pairs, a wave one pair at a time; the 27 kernel
+// (target group, component) pairs, a wave one pair at a time; the 27 kernel
 // values of a frequency are in LDS (the 13 with a leading negative offset are
-// the conjugates of their opposites: the point kernel is even).  Products and
+// the conjugates of their opposites: the point kernel is even), and a row of
+// zeros for the targets of a group that a source does not reach.  Products and
 // sums are FP64 for either storage type.  The workgroups that share a chunk
 // of frequencies are neighbours on one XCD: a source's line is read from
-// memory once and by its other targets from that L2, whose rate bounds it: 18 GB
-// in 1.2 ms for the 7411 parent pairs of a 4290-block solve in FP64.
+// memory once, and by its other groups from that L2.  Four targets share a
+// load of a source (2.2 targets on average in a 4290-block tree; 1.8 products
+// are issued for each that counts); skipping the others by a branch each put
+// an LDS wait into every branch.  One target a wave: 1.19 ms a solve of 4290
+// blocks in FP64, 2.28 for three components in FP32; four: 1.06 and 1.83
+// (branches: 1.07 and 2.04).  The spectra read and written once are 0.54 and
+// 0.80 ms of that at the rate of a copy.
 // ---------------------------------------------------------------------------
 constexpr int kMacWaves = 8;
 
 template<int U, class T>
-__device__ inline void mac_entries(const int* __restrict__ ent, int& e, int end,
-    const typename Spec<T>::C* __restrict__ sp, const double2* Gs, double2& acc)
+__device__ inline void mac_entries(const int2* __restrict__ ent, int& e, int end,
+    const typename Spec<T>::C* __restrict__ sp, const double2* Gs, double2 (&acc)[4])
 {
     for (; e + U <= end; e += U)
     {
-        int                 id[U];
+        int2                id[U];
         typename Spec<T>::C S[U];
 #pragma unroll
         for (int i = 0; i < U; ++i) id[i] = ent[e + i];
 #pragma unroll
-        for (int i = 0; i < U; ++i) S[i] = sp[(id[i] >> 5) * 64];
+        for (int i = 0; i < U; ++i) S[i] = sp[(size_t)id[i].x * 64];
 #pragma unroll
-        for (int i = 0; i < U; ++i) cfma(Spec<T>::get(S[i]), Gs[(id[i] & 31) * 64], acc);
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) cfma(Spec<T>::get(S[i]), Gs[((id[i].y >> 8 * t) & 255) * 64], acc[t]);
     }
 }
 
 template<class T>
-__global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int* __restrict__ begin,
-    const int* __restrict__ ent, int ntgt, int nsrc, int ncomp, const double2* __restrict__ ghat,
+__global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int4* __restrict__ group,
+    const int* __restrict__ begin, const int2* __restrict__ ent, int ngroup, int ntgt, int nsrc, int ncomp, const double2* __restrict__ ghat,
     const typename Spec<T>::C* __restrict__ sspec, typename Spec<T>::C* __restrict__ tspec, int nchunk, int nseg)
 {
-    __shared__ double2 Gs[27 * 64];
+    __shared__ double2 Gs[(kParentNone + 1) * 64];
     const int          r = blockIdx.x >> 3, chunk = (r / nseg) * 8 + (blockIdx.x & 7), seg = r % nseg;
     if (chunk >= nchunk) return;  // the whole workgroup
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wave == kMacWaves - 1) Gs[kParentNone * 64 + lane] = make_double2(0.0, 0.0);
     for (int o = wave; o < 27; o += kMacWaves)
     {
         // stored: offsets 13 (own parent) to 26; offset o < 13 is the opposite of 26 - o
@@ -476,18 +485,25 @@ __global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int* __rest
         Gs[o * 64 + lane] = g;
     }
     __syncthreads();
-    const int npair = ntgt * ncomp, per = (npair + nseg - 1) / nseg, lo = seg * per, hi = min(lo + per, npair);
+    const int npair = ngroup * ncomp, per = (npair + nseg - 1) / nseg, lo = seg * per, hi = min(lo + per, npair);
     for (int pr = lo + wave; pr < hi; pr += kMacWaves)
     {
-        const int c = pr / ntgt, t = pr - c * ntgt;
-        const int end = begin[t + 1];
-        int       e = begin[t];
+        const int  c = pr / ngroup, g = pr - c * ngroup;
+        const int  end = begin[g + 1];
+        int        e = begin[g];
+        const int4 to = group[g];
         const typename Spec<T>::C* sp = sspec + ((size_t)chunk * ncomp + c) * nsrc * 64 + lane;
-        double2   acc = make_double2(0.0, 0.0);
-        mac_entries<9, T>(ent, e, end, sp, Gs + lane, acc);
-        mac_entries<3, T>(ent, e, end, sp, Gs + lane, acc);
+        typename Spec<T>::C*       tp = tspec + ((size_t)chunk * ncomp + c) * ntgt * 64 + lane;
+        double2 acc[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = make_double2(0.0, 0.0);
+        mac_entries<8, T>(ent, e, end, sp, Gs + lane, acc);
+        mac_entries<2, T>(ent, e, end, sp, Gs + lane, acc);
         mac_entries<1, T>(ent, e, end, sp, Gs + lane, acc);
-        tspec[(((size_t)chunk * ncomp + c) * ntgt + t) * 64 + lane] = Spec<T>::put(acc);
+        if (to.x >= 0) tp[(size_t)to.x * 64] = Spec<T>::put(acc[0]);
+        if (to.y >= 0) tp[(size_t)to.y * 64] = Spec<T>::put(acc[1]);
+        if (to.z >= 0) tp[(size_t)to.z * 64] = Spec<T>::put(acc[2]);
+        if (to.w >= 0) tp[(size_t)to.w * 64] = Spec<T>::put(acc[3]);
     }
 }
 
@@ -724,11 +740,13 @@ struct Run
             src, b.fstride, p.src_child, p.nsrc, b.k, p.mid);
         hipLaunchKernelGGL((k_parent_fwd_plane<N, T>), dim3((unsigned)(ns * G::H)), dim3(G::T), 0, s, p.mid, (C*)p.sspec,
             (int)ns);
-        // four (target, component) pairs a wave: fewer read the kernel values more often, more leave a
-        // chunk's sources to L2 for longer (1, 3, 8 pairs: 1.31, 1.19, 1.22 ms a solve of 4290 blocks)
-        const int nchunk = G::NCH, nseg = (int)std::min(64L, (nt + 4 * kMacWaves - 1) / (4 * kMacWaves));
+        // (group, component) pairs a wave: fewer read the kernel values more often, more leave a chunk's
+        // sources to L2 for longer (4290 blocks, 2 and 4 pairs: FP64 1.058 and 1.065 ms, with fewer blocks
+        // 0.389 and 0.404; FP32, three components, 1.95 and 1.83)
+        constexpr int kRun = sizeof(T) == 8 ? 2 : 4;
+        const int nchunk = G::NCH, nseg = (int)std::min(64L, ((long)p.ngroup * b.k + kRun * kMacWaves - 1) / (kRun * kMacWaves));
         hipLaunchKernelGGL(k_parent_mac<T>, dim3((unsigned)((nchunk + 7) / 8 * 8 * nseg)), dim3(64 * kMacWaves), 0, s,
-            p.begin, p.entries, p.ntgt, p.nsrc, b.k, p.ghat, (const C*)p.sspec, (C*)p.tspec, nchunk, nseg);
+            p.group, p.begin, p.entries, p.ngroup, p.ntgt, p.nsrc, b.k, p.ghat, (const C*)p.sspec, (C*)p.tspec, nchunk, nseg);
         hipLaunchKernelGGL(
             (k_parent_inv_plane<N, T>), dim3((unsigned)(nt * G::H)), dim3(G::T), 0, s, (const C*)p.tspec, p.mid,
             (int)nt);
