@@ -480,10 +480,8 @@ void GpuSolver::reserve_components(int k)
         a->alloc(fs);
         IBLGF_HIP(hipMemset(a->p, 0, fs * sizeof(double)));
     }
-    w.sspec.alloc(ss);
+    w.sspec.alloc(ss);  // (a pass reads no spectrum that it has not written)
     w.tspec.alloc(ss);
-    IBLGF_HIP(hipMemset(w.sspec.p, 0, ss * sizeof(double2)));
-    IBLGF_HIP(hipMemset(w.tspec.p, 0, ss * sizeof(double2)));
     w.k = k;
     work_ = std::move(w);
     wp_ = WorkPtrs{work_.src.p, work_.tgt.p, work_.fmm_s.p, work_.fmm_t.p, work_.sspec.p, work_.tspec.p};
@@ -1143,16 +1141,15 @@ const double2* GpuSolver::parent_ghat()
     if (par_ghat_.n > 0) return par_ghat_.p;
     const ParentGeo  g = launch::parent_geo(n_);
     const size_t     nf = static_cast<size_t>(g.H) * g.P * g.P;
-    DevArray<double> sample;
-    sample.alloc(static_cast<size_t>(14) * g.P * g.P * g.P);
-    DevArray<double2> a, b, gh;
-    a.alloc(14 * nf);
-    b.alloc(14 * nf);
+    const size_t     nsample = static_cast<size_t>(14) * g.P * g.P * g.P;
+    if (gen_sample_.n < nsample) gen_sample_.alloc(nsample);
+    if (gen_a_.n < 14 * nf) gen_a_.alloc(14 * nf);
+    if (gen_b_.n < 14 * nf) gen_b_.alloc(14 * nf);
+    DevArray<double2> gh;
     gh.alloc(14 * static_cast<size_t>(g.NF));
-    launch::parent_sample(stream_, n_, d_lgf_table_.p, lgf_nmax_, sample.p);
-    launch::parent_spectra(stream_, n_, sample.p, a.p, b.p, gh.p);
+    launch::parent_sample(stream_, n_, d_lgf_table_.p, lgf_nmax_, gen_sample_.p);
+    launch::parent_spectra(stream_, n_, gen_sample_.p, gen_a_.p, gen_b_.p, gh.p);
     IBLGF_HIP(hipGetLastError());
-    sync();  // the scratch is released on return
     par_ghat_ = std::move(gh);
     return par_ghat_.p;
 }
