@@ -6,7 +6,7 @@
 // Every operation of the step is a launch on the solver stream: the field
 // operations stream whole blocks (HBM-bound), the stencils read the one-cell
 // buffers that a halo fill refreshed, and the solves are the FMM path.  With
-// graphs on, the step (about 400 launches on a 4000-block tree) is captured
+// graphs on, the step (255 launches on a 403-block tree) is captured
 // once per (fields, dt, Re, frame) and replayed as one graph.
 #include "gpu_solver.hpp"
 #include "kernels.hpp"

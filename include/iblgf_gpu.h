@@ -396,8 +396,10 @@ int iblgf_gpu_stream(iblgf_gpu_ctx* ctx, void** stream);
 /* Kernel-class timing with HIP events on the context's stream, in place of
  * the reference's POISSON_TIMINGS / Fmm::Timings clocks
  * (include/iblgf/solver/poisson/poisson.hpp:621-893; include/iblgf/fmm/fmm.hpp:1197-1240).
- * Classes: 0 forward DFT, 1 spectral MAC, 2 inverse DFT, 3 transfers,
- * 4 other.  read() synchronises, then returns per class the summed event
+ * Classes: 0 forward DFT and 2 inverse DFT (block transforms), 1 spectral MAC
+ * (block products, and the finest level of a Laplace pass as a whole: its
+ * transforms and products of whole parents), 3 transfers, 4 other (the
+ * separable integrating-factor sums among them).  read() synchronises, then returns per class the summed event
  * time (ms), the number of timed launches and the work units (blocks for
  * 0/2, source-target pairs for 1, parent-child transfers for 3). */
 int iblgf_gpu_timing_enable(iblgf_gpu_ctx* ctx, int enable);
@@ -722,8 +724,8 @@ int iblgf_gpu_helm2d_table(const double* c, int nmodes, int nx, int ny, double* 
  * block pair of one level, include/iblgf/utilities/convolution.hpp:259-260
  * with the Helmholtz kernel):
  *   dst[k][t] = scale * sum_s table[k][|tj - sj|][|ti - si|] * src[k][s],
- * summed directly over every cell s of the patch (so dst satisfies
- * (Lap_h - c^2) dst = scale * src at interior cells).  src and dst (nmodes x
+ * the sum over every cell s of the patch, directly or by transforms along x
+ * (so dst satisfies (Lap_h - c^2) dst = scale * src at interior cells).  src and dst (nmodes x
  * ny x nx doubles) must differ; same limits as iblgf_gpu_helm2d_table. */
 int iblgf_gpu_helm2d_convolve(
     const double* table, int nmodes, int nx, int ny, const double* src, double* dst, double scale, void* stream);
