@@ -45,6 +45,14 @@ def test_uniform_regions(oracle_mod, extent, region):
     _check(oracle_mod, _uniform(extent, region), 1, PREC_FP64, 1e-12)
 
 
+@pytest.mark.parametrize("extent, precision, bound", [(6, PREC_FP64, 1e-12), (8, PREC_FP64, 1e-12), (6, PREC_MIXED, 1e-6)])
+def test_groups_of_targets(oracle_mod, extent, precision, bound):
+    """4 x 3 x 2 parents: groups of four targets, of two, and shared sources
+    that reach some of a group only."""
+    print(f"case: whole-parent products in groups, {extent}^3 blocks, precision {precision}", flush=True)
+    _check(oracle_mod, _uniform(extent, (7, 5, 3), box=16), 2, precision, bound)
+
+
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED, PREC_FP16X3_FORWARD])
 @pytest.mark.parametrize("extent", [6, 10])
 def test_adaptive_tree_two_components(oracle_mod, extent, precision):
