@@ -1124,14 +1124,15 @@ void GpuSolver::set_precision(int p)
 void GpuSolver::prepare_laplace()
 {
     for (int l = base_level_; l < depth_; ++l)
-        for (int nl = 0; nl < 2; ++nl)
-        {
-            PassPlan& p = pass(l, nl, false);
-            for (auto& m : p.mac) ghat(true, m.d, 0.0);
-            if (p.npar_tgt > 0) parent_ghat();
-        }
+        for (int nl = 0; nl < 2; ++nl) prepare_pass(pass(l, nl, false));
     reserve_parents();
     sync();
+}
+
+void GpuSolver::prepare_pass(PassPlan& p)
+{
+    for (auto& m : p.mac) ghat(true, m.d, 0.0);
+    if (p.npar_tgt > 0) parent_ghat();
 }
 
 // Kernel spectra of the whole-parent transforms (level difference

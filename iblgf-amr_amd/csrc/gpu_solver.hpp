@@ -358,6 +358,7 @@ class GpuSolver
     static int pass_key(int L, int idx, bool neighbor_only) { return (L * 64 + idx) * 2 + (neighbor_only ? 1 : 0); }
     bool      has_ghat(bool laplace, int d, double alpha) const;
     void      build_separable(PassPlan& p, std::vector<char>& done);
+    void      prepare_pass(PassPlan& p);  // kernel spectra of one Laplace pass
     void      reserve_parents();
     const double2* parent_ghat();
     void      run_parents(PassPlan& p, double scale, const Batch& b);

@@ -376,9 +376,9 @@ void GpuSolver::step_prepare(const double alpha[3], int refresh)
     if (std::fabs(alpha[2]) > 1e-14) prepare_if(alpha[2]);
     if (refresh)
     {
-        // the STREAM pass and its kernel spectra
-        PassPlan& sp = pass_idx(base_level_, fmm_mask_idx_gen(MASK_STREAM), false);
-        for (auto& m : sp.mac) ghat(true, m.d, 0.0);
+        // the STREAM pass: it can have more parents than any pass of the solves
+        prepare_pass(pass_idx(base_level_, fmm_mask_idx_gen(MASK_STREAM), false));
+        reserve_parents();
         if (refresh == 1) prepare_if(0.0);
         sync();
     }

@@ -135,6 +135,29 @@ def test_step_graph_replays_equal_eager():
     s.set_graphs(False)
 
 
+def test_refresh_first_met_with_graphs_on():
+    """The first step with the velocity refresh comes after one without, both
+    captured: on this tree the refresh's STREAM pass has 512 source parents and
+    the passes prepared before it at most 511, so whatever it needs beyond
+    theirs has to be there before its capture starts."""
+    print("case: a captured step without the velocity refresh, then one with it", flush=True)
+    tree = setups.VortexRings(seed=7, base_blocks=16, block_extent=6, nref=1, nrings=1, centre_range=2.0,
+                              radius=(5.0, 6.0), core=(1.5, 2.0), refinement_factor=0.1).tree
+    u0 = setups.GaussianFlow(tree, BLOBS).velocity()
+
+    def steps(graphs):
+        s = PoissonSolver(tree)
+        s.set_graphs(graphs)
+        fu = [s.field() for _ in range(3)]
+        for f, x in zip(fu, u0):
+            s.upload(f, x)
+        for refresh in (0, 1, 2):
+            s.ifherk_step(fu, 2e-4, 500.0, refresh=refresh)
+        return [s.download(f) for f in fu]
+
+    assert all(np.array_equal(g, r) for g, r in zip(steps(True), steps(False)))
+
+
 def test_step_refuses_bad_arguments():
     from iblgf_amd import IBLGF_ERR_ARG, IblgfError
 
