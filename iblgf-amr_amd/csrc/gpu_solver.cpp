@@ -286,8 +286,8 @@ void GpuSolver::upload_forest(const std::vector<const Octree*>& trees)
     fields_.clear();
     drop_graphs();
     work_ = Work{};
-    par_need_s_ = par_need_t_ = par_need_m_ = 0;
-    for (DevArray<double2>* a : {&par_sspec_, &par_tspec_, &par_mid_}) *a = DevArray<double2>{};
+    par_extra_ = DevArray<double2>{};
+    par_one_ = DevArray<double2>{};
     reserve_components(1);
 
     // solver-level block lists
@@ -467,24 +467,25 @@ FieldTable GpuSolver::work_table(double* base, int k) const
     return t;
 }
 
+static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
+
 void GpuSolver::reserve_components(int k)
 {
     if (k < 1 || k > kMaxComponents) throw std::invalid_argument("component count out of range");
     if (k <= work_.k) return;
     if (stream_) sync();  // solves in flight still use the old arrays
     drop_graphs();        // captured graphs point at the old arrays
-    const size_t fs = field_size() * k, ss = static_cast<size_t>(nb_) * nf_ * k;
+    const size_t fs = field_size() * k, ss = round256(static_cast<size_t>(nb_) * nf_ * k * sizeof(double2));
     Work w;
     for (DevArray<double>* a : {&w.src, &w.tgt, &w.fmm_s, &w.fmm_t})
     {
         a->alloc(fs);
         IBLGF_HIP(hipMemset(a->p, 0, fs * sizeof(double)));
     }
-    w.sspec.alloc(ss);  // (a pass reads no spectrum that it has not written)
-    w.tspec.alloc(ss);
+    w.spec.alloc(2 * ss / sizeof(double2));  // (a pass reads no spectrum that it has not written)
     w.k = k;
     work_ = std::move(w);
-    wp_ = WorkPtrs{work_.src.p, work_.tgt.p, work_.fmm_s.p, work_.fmm_t.p, work_.sspec.p, work_.tspec.p};
+    wp_ = WorkPtrs{work_.src.p, work_.tgt.p, work_.fmm_s.p, work_.fmm_t.p, work_.spec.p, 2 * ss};
 }
 
 Batch GpuSolver::batch(int k) const
@@ -856,12 +857,6 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
             p.par_ent.upload(pent);
             p.par_npairs = p.par_stats.npairs = p.par_stats.pairs_full = pairs_parents;
             p.par_stats.nentries = p.par_stats.nfull = entries_parents;
-            const ParentGeo g = launch::parent_geo(n_);
-            const size_t    nf = g.NF;
-            par_need_s_ = std::max(par_need_s_, p.npar_src * nf);
-            par_need_t_ = std::max(par_need_t_, p.npar_tgt * nf);
-            par_need_m_ = std::max({par_need_m_, static_cast<size_t>(p.npar_src) * g.H * g.M * g.M,
-                static_cast<size_t>(p.npar_tgt) * g.H * g.W * g.W});
             p.npairs += pairs_parents;
             pairs_here -= pairs_parents;
         }
@@ -926,6 +921,8 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
     for (size_t i = p.nfwd_coarse; i < fwd.size(); ++i)
         if (fwd[i] >= lvl_begin_[L + 1]) throw std::logic_error("pass plan: sources finer than the pass level");
     p.inv.upload(inv);
+    for (const std::vector<int>* l : {&fwd, &inv})
+        for (int slot : *l) p.spec_slots = std::max(p.spec_slots, slot + 1);
     p.ninv_top = 0;
     while (p.ninv_top < static_cast<int>(inv.size()) && inv[p.ninv_top] >= lvl_begin_[L] &&
            inv[p.ninv_top] < lvl_begin_[L + 1])
@@ -1121,11 +1118,23 @@ void GpuSolver::set_precision(int p)
     precision_ = p;
 }
 
-void GpuSolver::prepare_laplace()
+void GpuSolver::prepare_laplace(int k)
 {
     for (int l = base_level_; l < depth_; ++l)
-        for (int nl = 0; nl < 2; ++nl) prepare_pass(pass(l, nl, false));
-    reserve_parents();
+        for (int nl = 0; nl < 2; ++nl)
+        {
+            PassPlan& p = pass(l, nl, false);
+            prepare_pass(p);
+            reserve_parents(p, k);
+        }
+    // What an allocation-free solve needs beyond its region: of a size that
+    // holds in every precision, and kept while the tree is loaded.
+    size_t one = 0;
+    for (const auto& kv : passes_)
+        if (kv.second->npar_tgt > 0 && amr2amr(*kv.second) && !fits_region(*kv.second))
+            one = std::max(one, launch::parent_bytes(n_, kPrecFp64, kv.second->npar_src, kv.second->npar_tgt, 0));
+    if (par_one_.n == 0 && one > 0 && region_bytes(kPrecMixed) <= kNoallocScratchBytes)
+        par_one_.alloc(one / sizeof(double2));
     sync();
 }
 
@@ -1155,27 +1164,77 @@ const double2* GpuSolver::parent_ghat()
     return par_ghat_.p;
 }
 
-// Scratch of the whole-parent transforms for every pass built so far and the
-// component count of the work arrays.
-void GpuSolver::reserve_parents()
+// What the block spectra of a pass (slots below spec_slots: coarser levels,
+// and level-L blocks that are not part of whole parents) leave of the spectra's
+// memory, `spec` of `bytes`, when they lie at its start: the whole parents' scratch.
+GpuSolver::SpecPtrs GpuSolver::spectra(const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes) const
 {
-    const size_t k = static_cast<size_t>(work_.k);
-    if (par_sspec_.n >= par_need_s_ * k && par_tspec_.n >= par_need_t_ * k && par_mid_.n >= par_need_m_ * k) return;
-    sync();         // passes in flight still use the old arrays
-    drop_graphs();  // captured graphs point at the old arrays
-    if (par_sspec_.n < par_need_s_ * k) par_sspec_.alloc(par_need_s_ * k);
-    if (par_tspec_.n < par_need_t_ * k) par_tspec_.alloc(par_need_t_ * k);
-    if (par_mid_.n < par_need_m_ * k) par_mid_.alloc(par_need_m_ * k);
+    const size_t elem = prec == kPrecFp64 ? sizeof(double2) : sizeof(float2);
+    const size_t half = p.npar_tgt > 0 ? round256(static_cast<size_t>(p.spec_slots) * nf_ * b.k * elem) : bytes / 2;
+    char*        at = static_cast<char*>(spec);
+    SpecPtrs     s{at, at + half, at + 2 * half, bytes - 2 * half, b};
+    if (p.npar_tgt > 0) s.b.sstride = static_cast<long>(p.spec_slots) * nf_;
+    return s;
 }
 
-void GpuSolver::run_parents(PassPlan& p, double scale, const Batch& b)
+static bool parents_fit(int n, int prec, const PassPlan& p, int k, size_t room)
 {
-    const double2* g = parent_ghat();
-    reserve_parents();
-    const ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_group.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt,
-        static_cast<int>(p.par_group.n), g,
-        par_sspec_.p, par_tspec_.p, par_mid_.p};
-    launch::parent_pass(stream_, n_, precision_, pp, wp_.src, wp_.tgt, scale, b);
+    return room > 0 && launch::parent_bytes(n, prec, static_cast<long>(p.npar_src) * k,
+                           static_cast<long>(p.npar_tgt) * k, room) > 0;
+}
+
+// Whether the whole parents of a pass fit the region of an allocation-free
+// solve in every precision.
+bool GpuSolver::fits_region(const PassPlan& p) const
+{
+    for (int prec : {kPrecFp64, kPrecMixed})
+    {
+        const size_t sb = spec_region_bytes(prec);
+        if (!parents_fit(n_, prec, p, 1, spectra(p, prec, batch(1), nullptr, 2 * sb).rest_bytes)) return false;
+    }
+    return true;
+}
+
+// The passes of the AMR2AMR solves.
+bool GpuSolver::amr2amr(const PassPlan& p) const { return !p.neighbor_only && p.idx >= 15 && p.idx < 30; }
+
+// Scratch of a pass of k components whose whole parents do not fit beside its
+// block spectra even in rounds (few and partly filled parents), for all of
+// their frequencies at once.
+void GpuSolver::reserve_parents(const PassPlan& p, int k)
+{
+    if (p.npar_tgt == 0) return;
+    const size_t bytes = 2 * round256(static_cast<size_t>(nb_) * nf_ * std::max(k, work_.k) * sizeof(double2));
+    if (parents_fit(n_, precision_, p, k, spectra(p, precision_, batch(k), nullptr, bytes).rest_bytes)) return;
+    const size_t need = launch::parent_bytes(
+        n_, precision_, static_cast<long>(p.npar_src) * k, static_cast<long>(p.npar_tgt) * k, 0);
+    if (par_extra_.n * sizeof(double2) >= need) return;
+    sync();         // passes in flight still use the old array
+    drop_graphs();  // captured graphs point at it
+    par_extra_.alloc(need / sizeof(double2));
+}
+
+void GpuSolver::run_parents(PassPlan& p, double scale, const SpecPtrs& sp)
+{
+    ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_group.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt,
+        static_cast<int>(p.par_group.n), parent_ghat(), sp.rest, sp.rest_bytes};
+    if (wp_.region)
+    {
+        // nothing but the region, the plans and what prepare has put aside
+        if (!fits_region(p))
+        {
+            if (!par_one_.p) throw std::logic_error("whole parents: no scratch beside the region");
+            pp.scratch = par_one_.p;
+            pp.bytes = par_one_.n * sizeof(double2);
+        }
+    }
+    else if (!parents_fit(n_, precision_, p, sp.b.k, sp.rest_bytes))
+    {
+        reserve_parents(p, sp.b.k);
+        pp.scratch = par_extra_.p;
+        pp.bytes = par_extra_.n * sizeof(double2);
+    }
+    launch::parent_pass(stream_, n_, precision_, pp, wp_.src, wp_.tgt, scale, sp.b);
 }
 
 void GpuSolver::prepare_if(double alpha_base)
@@ -1195,8 +1254,10 @@ void GpuSolver::prepare_if(double alpha_base)
 int GpuSolver::forward_legs() const { return precision_ == kPrecF16x3Forward ? kPrecF16x3 : precision_; }
 int GpuSolver::inverse_legs() const { return precision_ == kPrecF16x3Forward ? kPrecMixed : precision_; }
 
-void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& b)
+void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& batch)
 {
+    const SpecPtrs sp = spectra(p, precision_, batch, wp_.spec, wp_.spec_bytes);
+    const Batch&   b = sp.b;
     double*      fmm_s = wp_.fmm_s;
     double*      fmm_t = wp_.fmm_t;
     const int    L = p.L;
@@ -1208,7 +1269,7 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
     {
         const double* iv = if_iv(alpha);
         timer_.begin(stream_);
-        launch::if_separable(stream_, n_, wp_.src, static_cast<double*>(wp_.sspec), wp_.tgt, p.sep_z.p,
+        launch::if_separable(stream_, n_, wp_.src, static_cast<double*>(wp_.spec), wp_.tgt, p.sep_z.p,
             p.sep_z.size() / 3, p.sep_t.p, p.sep_t.size() / 10, iv, b, b.sstride);
         timer_.end(stream_, KC_OTHER, 0);
     }
@@ -1248,15 +1309,15 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
     if (p.npar_tgt > 0)
     {
         timer_.begin(A);
-        run_parents(p, scale, b);
+        run_parents(p, scale, sp);
         timer_.end(A, KC_MAC, p.par_npairs * b.k);
     }
     const int nfine = static_cast<int>(p.fwd.size()) - p.nfwd_coarse;
     timer_.begin(A);
-    launch::forward_dft(A, n_, forward_legs(), fmm_s, p.fwd.p + p.nfwd_coarse, nfine, wp_.sspec, b, wp_.src, 0);
+    launch::forward_dft(A, n_, forward_legs(), fmm_s, p.fwd.p + p.nfwd_coarse, nfine, sp.sspec, b, wp_.src, 0);
     timer_.end(A, KC_FORWARD, static_cast<long>(nfine) * b.k);
     timer_.begin(B);
-    launch::forward_dft(B, n_, forward_legs(), fmm_s, p.fwd.p, p.nfwd_coarse, wp_.sspec, b);
+    launch::forward_dft(B, n_, forward_legs(), fmm_s, p.fwd.p, p.nfwd_coarse, sp.sspec, b);
     timer_.end(B, KC_FORWARD, static_cast<long>(p.nfwd_coarse) * b.k);
     for (size_t i = 0; i < p.mac.size(); ++i)
     {
@@ -1264,17 +1325,17 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
         hipStream_t         s = m.lambda == L ? A : B;
         timer_.begin(s);
         launch::spectral_mac(s, n_, precision_, m.groups.p, m.groups.size(), m.srcs.p, m.rowoff.p, m.olist.p,
-            m.nused, m.compact, gh[i], wp_.sspec, wp_.tspec, b, m.queue.p);
+            m.nused, m.compact, gh[i], sp.sspec, sp.tspec, b, m.queue.p);
         timer_.end(s, KC_MAC, m.npairs * b.k);
     }
     // Level-L targets (first in inv) add into the target array, coarser ones
     // are written to fmm_t and interpolated down.
     const int ntop = p.ninv_top, nrest = static_cast<int>(p.inv.size()) - ntop;
     timer_.begin(A);
-    launch::inverse_dft(A, n_, inverse_legs(), wp_.tspec, p.inv.p, ntop, wp_.tgt, iscale, true, b);
+    launch::inverse_dft(A, n_, inverse_legs(), sp.tspec, p.inv.p, ntop, wp_.tgt, iscale, true, b);
     timer_.end(A, KC_INVERSE, static_cast<long>(ntop) * b.k);
     timer_.begin(B);
-    launch::inverse_dft(B, n_, inverse_legs(), wp_.tspec, p.inv.p + ntop, nrest, fmm_t, iscale, false, b);
+    launch::inverse_dft(B, n_, inverse_legs(), sp.tspec, p.inv.p + ntop, nrest, fmm_t, iscale, false, b);
     timer_.end(B, KC_INVERSE, static_cast<long>(nrest) * b.k);
     if (coarse)
     {
@@ -1405,7 +1466,7 @@ void GpuSolver::apply_lgf_batch(const int* src, const int* dst, int k, int mesh)
     mesh_ = mesh;
     try
     {
-        run_captured(key, [this] { prepare_laplace(); }, [this, src, dst, k] { lgf_batch_body(src, dst, k); });
+        run_captured(key, [this, k] { prepare_laplace(k); }, [this, src, dst, k] { lgf_batch_body(src, dst, k); });
     }
     catch (...)
     {
@@ -1496,7 +1557,7 @@ void GpuSolver::solve_sequence(const std::vector<SolveItem>& items)
         [this, &items] {
             for (const SolveItem& it : items)
             {
-                if (it.laplace) prepare_laplace();
+                if (it.laplace) prepare_laplace(static_cast<int>(it.src.size()));
                 else
                     prepare_if(it.alpha);
             }
@@ -1530,7 +1591,7 @@ std::string GpuSolver::autotune(const int* src, const int* dst, int k, bool lapl
 {
     if (reps < 1) throw std::invalid_argument("autotune: reps must be positive");
     check_batch(src, dst, k);
-    if (laplace) prepare_laplace();
+    if (laplace) prepare_laplace(k);
     else
         prepare_if(alpha_base);
     const bool graphs = graphs_, timing = timer_.enabled();
@@ -1635,21 +1696,21 @@ bool GpuSolver::prepared(bool laplace, double alpha_base) const
             if (it == passes_.end() || (!laplace && !if_iv_.count(alpha))) return false;
             for (const auto& m : it->second->mac)
                 if (!has_ghat(laplace, m.d, alpha)) return false;
-            if (it->second->npar_tgt > 0 && (par_ghat_.n == 0 || par_sspec_.n < par_need_s_ ||
-                                                par_tspec_.n < par_need_t_ || par_mid_.n < par_need_m_))
+            if (it->second->npar_tgt > 0 && (par_ghat_.n == 0 || (par_one_.n == 0 && !fits_region(*it->second))))
                 return false;
         }
     }
     return true;
 }
 
-static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
-
-size_t GpuSolver::region_bytes() const
+size_t GpuSolver::spec_region_bytes(int prec) const
 {
-    const size_t fb = round256(field_size() * sizeof(double));
-    const size_t sb = round256(static_cast<size_t>(nb_) * nf_ * (precision_ == 0 ? sizeof(double2) : sizeof(float2)));
-    return 4 * fb + 2 * sb;
+    return round256(static_cast<size_t>(nb_) * nf_ * (prec == kPrecFp64 ? sizeof(double2) : sizeof(float2)));
+}
+
+size_t GpuSolver::region_bytes(int prec) const
+{
+    return 4 * round256(field_size() * sizeof(double)) + 2 * spec_region_bytes(prec);
 }
 
 void GpuSolver::solve_in_region(int src, int dst, bool laplace, double alpha_base, void* region, size_t bytes)
@@ -1666,13 +1727,13 @@ void GpuSolver::solve_in_region(int src, int dst, bool laplace, double alpha_bas
     field_data(dst);
     IBLGF_HIP(hipSetDevice(device_));
     const size_t fb = round256(field_size() * sizeof(double));
-    const size_t sb = round256(static_cast<size_t>(nb_) * nf_ * (precision_ == 0 ? sizeof(double2) : sizeof(float2)));
     char*        p = static_cast<char*>(region);
     // The region keeps whatever the last user left in it.
     noalloc_clear(stream_, region, need);
     const WorkPtrs saved = wp_;
     wp_ = WorkPtrs{reinterpret_cast<double*>(p), reinterpret_cast<double*>(p + fb),
-        reinterpret_cast<double*>(p + 2 * fb), reinterpret_cast<double*>(p + 3 * fb), p + 4 * fb, p + 4 * fb + sb};
+        reinterpret_cast<double*>(p + 2 * fb), reinterpret_cast<double*>(p + 3 * fb), p + 4 * fb,
+        2 * spec_region_bytes(precision_), true};
     try
     {
         if (laplace) lgf_batch_body(&src, &dst, 1);

@@ -89,6 +89,7 @@ struct PassPlan
     DevArray<int4>                   par_group;
     DevArray<int2>                   par_ent;
     int                              npar_src = 0, npar_tgt = 0;
+    int                              spec_slots = 0;  // block spectra are of slots below this
     long                             par_nfwd = 0, par_ninv = 0, par_npairs = 0;
     MacLevelPlan                     par_stats;
     long                             npairs = 0;
@@ -230,7 +231,8 @@ class GpuSolver
     // (region_bytes() bytes, each part 256-byte aligned), which the solve
     // clears by kernel first.  Needs prepared(): every pass plan and kernel
     // spectrum of the solve built beforehand in the current precision.
-    size_t region_bytes() const;
+    size_t region_bytes() const { return region_bytes(precision_); }
+    size_t region_bytes(int prec) const;
     bool   prepared(bool laplace, double alpha_base) const;
     void   solve_in_region(int src, int dst, bool laplace, double alpha_base, void* region, size_t bytes);
     static constexpr int kMaxComponents = 64;
@@ -246,7 +248,7 @@ class GpuSolver
     void set_concurrency(bool on);
     bool graphs() const { return graphs_; }
     // Build the kernel spectra that a solve will use (cold-path work).
-    void prepare_laplace();
+    void prepare_laplace(int k = 1);  // for solves of up to k components
     void prepare_if(double alpha_base);
 
     // Finest-level solves with an immersed-boundary FMM mask (MASK_IB2xIB or
@@ -359,12 +361,11 @@ class GpuSolver
     bool      has_ghat(bool laplace, int d, double alpha) const;
     void      build_separable(PassPlan& p, std::vector<char>& done);
     void      prepare_pass(PassPlan& p);  // kernel spectra of one Laplace pass
-    void      reserve_parents();
+    void      reserve_parents(const PassPlan& p, int k);
     const double2* parent_ghat();
-    void      run_parents(PassPlan& p, double scale, const Batch& b);
     const double* if_iv(double alpha);
     const DevArray<int>& face_clean_list(int kind, int level, bool leaf_only);
-    void      run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& b);
+    void      run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& batch);
     void      lgf_batch_body(const int* src, const int* dst, int k);
     void      if_batch_body(const int* src, const int* dst, int k, double alpha_base);
     void      run_captured(const std::vector<int64_t>& key, const std::function<void()>& prepare,
@@ -419,13 +420,13 @@ class GpuSolver
     std::vector<DevArray<double>> fields_;
     std::vector<char>             field_f32_;
     // Work arrays of the solves, k components each, component-major
-    // (component c of a field array at c * field_size(), of a spectrum array
-    // at c * nb * NF): source and target temporaries, correction, the FMM
-    // pass's source/target and the source/target spectra.
+    // (component c of a field array at c * field_size()): source and target
+    // temporaries, correction, the FMM pass's source/target and the memory of
+    // the spectra, two complex values of FP64 a block, component and frequency.
     struct Work
     {
         DevArray<double>  src, tgt, fmm_s, fmm_t;
-        DevArray<double2> sspec, tspec;
+        DevArray<double2> spec;
         int               k = 0;
     };
     Work work_;
@@ -438,16 +439,28 @@ class GpuSolver
         double* tgt = nullptr;
         double* fmm_s = nullptr;
         double* fmm_t = nullptr;
-        void*   sspec = nullptr;
-        void*   tspec = nullptr;
+        void*   spec = nullptr;
+        size_t  spec_bytes = 0;
+        bool    region = false;
     };
     WorkPtrs wp_;
-    // Scratch of the whole-parent transforms, for the largest pass built and
-    // work_.k components: spectra of source and target parents and the
-    // half-transformed columns between the kernels.  A context's own, so an
-    // allocation-free solve finds it after prepare.
-    DevArray<double2> par_sspec_, par_tspec_, par_mid_;
-    size_t            par_need_s_ = 0, par_need_t_ = 0, par_need_m_ = 0;  // of one component
+    // The spectra of one pass within that memory: source and target spectra of
+    // blocks, component c at c * b.sstride, and the rest.
+    struct SpecPtrs
+    {
+        void * sspec, *tspec, *rest;
+        size_t rest_bytes;
+        Batch  b;
+    };
+    void     run_parents(PassPlan& p, double scale, const SpecPtrs& sp);
+    SpecPtrs spectra(const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes) const;
+    bool     fits_region(const PassPlan& p) const;
+    bool     amr2amr(const PassPlan& p) const;
+    size_t   spec_region_bytes(int prec) const;
+    // Scratch of whole parents that do not fit the rest: of the largest such
+    // pass run, and (never moved while the tree is loaded) of the allocation-free
+    // solve's.
+    DevArray<double2> par_extra_, par_one_;
     DevArray<double2> par_ghat_;
     bool                                          graphs_ = false;
     std::map<std::vector<int64_t>, hipGraphExec_t> graph_cache_;

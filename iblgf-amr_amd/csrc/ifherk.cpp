@@ -377,8 +377,9 @@ void GpuSolver::step_prepare(const double alpha[3], int refresh)
     if (refresh)
     {
         // the STREAM pass: it can have more parents than any pass of the solves
-        prepare_pass(pass_idx(base_level_, fmm_mask_idx_gen(MASK_STREAM), false));
-        reserve_parents();
+        PassPlan& sp = pass_idx(base_level_, fmm_mask_idx_gen(MASK_STREAM), false);
+        prepare_pass(sp);
+        reserve_parents(sp, 1);
         if (refresh == 1) prepare_if(0.0);
         sync();
     }

@@ -120,9 +120,8 @@ struct ParentGeo
 // parent, offset (ox + 1) + 3 (oy + 1) + 9 (oz + 1) of the source from target
 // t of the group in byte t (kParentNone: not a source of that target)}, every
 // target's offsets ascending.
-// ghat: 14 spectra of parent_spectra (offsets 13 to 26).  Scratch for k components: sspec and
-// tspec a spectrum per source / target parent (FP64, or FP32 with prec > 0),
-// mid H values a column for the larger of nsrc M M and ntgt W W columns.
+// ghat: 14 spectra of parent_spectra (offsets 13 to 26).  scratch: `bytes` in
+// which parent_bytes finds room for the pass.
 constexpr int kParentNone = 27;  // a row of zeros
 struct ParentPass
 {
@@ -133,9 +132,8 @@ struct ParentPass
     const int2*    entries;
     int            nsrc, ntgt, ngroup;
     const double2* ghat;
-    void*          sspec;
-    void*          tspec;
-    double2*       mid;
+    void*          scratch;
+    size_t         bytes;
 };
 
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup i of a launch to
@@ -261,6 +259,12 @@ ParentGeo parent_geo(int n);
 // dst[target block] += scale * (every point's sum over the sources' interiors).
 void parent_pass(hipStream_t s, int n, int prec, const ParentPass& p, const double* src, double* dst, double scale,
     const Batch& b);
+// Scratch of a pass with nsrc source and ntgt target parents (times the
+// components), FP64 or (prec > 0) FP32 spectra: with room 0 the bytes for all
+// frequencies at once; otherwise the bytes it takes of `room`, in rounds of
+// fewer frequencies if need be, or 0 where even one plane a round does not
+// fit.  Results do not depend on it.
+size_t parent_bytes(int n, int prec, long nsrc, long ntgt, size_t room);
 // sample: 14 P^3 values; a, b: scratch of 14 H P P values each; ghat: 14 NF.
 void parent_sample(hipStream_t s, int n, const double* g, int nmax, double* sample);
 void parent_spectra(hipStream_t s, int n, const double* sample, double2* a, double2* b, double2* ghat);

@@ -288,10 +288,20 @@ constexpr int kLineThreads = 256;
 // Spectra are stored by chunks of 64 frequencies, in a chunk by parent: the
 // products read a chunk's sources from one stretch of memory.  (Parent by
 // parent, their rows of 1 KB lay 2 MB apart at n = 18: twice the time.)
-__device__ inline size_t spec_at(int f, int row, int rows)
+// chunk0: the first chunk that is stored.
+__device__ inline size_t spec_at(int f, int chunk0, int row, int rows)
 {
-    return ((size_t)(f >> 6) * rows + row) * 64 + (f & 63);
+    return ((size_t)((f >> 6) - chunk0) * rows + row) * 64 + (f & 63);
 }
+
+// The kz planes [z0, z0 + nz) of one round of a pass and the chunks they lie
+// in.  Frequencies are independent of each other between the z legs, so a
+// pass whose spectra do not fit its scratch takes them some planes at a time;
+// an outer chunk's other planes are neither written nor read.
+struct Slice
+{
+    int z0, nz, chunk0, nchunk;
+};
 
 // ---------------------------------------------------------------------------
 // Forward z leg (real to half spectrum): mid[item][kz][y][x], item = component
@@ -300,10 +310,11 @@ __device__ inline size_t spec_at(int f, int row, int rows)
 // absent child is zero).  Real input: k1 and R1 - k1 give conjugate
 // frequencies, so only k1 <= R1 / 2 is computed.  Memory bounds it: 0.65 GB in
 // 0.13 ms a 4290-block solve (a dense matrix from scalar registers: 0.32 ms).
+// PART: only planes [z0, z0 + nz) are kept; otherwise all H of them.
 // ---------------------------------------------------------------------------
-template<int N>
+template<int N, bool PART>
 __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __restrict__ src, long fcs,
-    const int* __restrict__ child, int count, int ncomp, double2* __restrict__ mid)
+    const int* __restrict__ child, int count, int ncomp, double2* __restrict__ mid, int z0, int nz)
 {
     using G = Par<N>;
     constexpr int E = G::E, M = G::M, MM = M * M, R1 = G::R1, R2 = G::R2, P = G::P, h = (R2 - 1) / 2;
@@ -319,7 +330,12 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __r
     for (int a = 0; a < E; ++a) in[a] = lo >= 0 ? src[(size_t)lo * G::N3 + a * G::NN] : 0.0;
 #pragma unroll
     for (int a = 0; a < E; ++a) in[E + a] = hi >= 0 ? src[(size_t)hi * G::N3 + a * G::NN] : 0.0;
-    double2* out = mid + (size_t)item * G::H * MM + col;
+    double2*   out = mid + (size_t)item * (PART ? nz : G::H) * MM + col;
+    const auto put = [&](int k, double2 X) {
+        if (!PART) out[(size_t)k * MM] = X;
+        else if (k >= z0 && k < z0 + nz)
+            out[(size_t)(k - z0) * MM] = X;
+    };
 #pragma unroll
     for (int k1 = 0; 2 * k1 <= R1; ++k1)
     {
@@ -346,7 +362,7 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __r
                 u[R2 - j] = d;
                 s0 += t;
             }
-            out[(size_t)kCrt<R1, R2>.k[k1][0] * MM] = make_double2(s0, 0.0);
+            put(kCrt<R1, R2>.k[k1][0], make_double2(s0, 0.0));
 #pragma unroll
             for (int k2 = 1; k2 <= h; ++k2)
             {
@@ -358,9 +374,9 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __r
                     D = fma(kRoots<R2>.s[(j * k2) % R2], u[R2 - j], D);
                 }
                 const int k = kCrt<R1, R2>.k[k1][k2];
-                if (k < G::H) out[(size_t)k * MM] = make_double2(C, -D);
+                if (k < G::H) put(k, make_double2(C, -D));
                 else
-                    out[(size_t)(P - k) * MM] = make_double2(C, D);
+                    put(P - k, make_double2(C, D));
             }
         }
         else
@@ -381,9 +397,9 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __r
             }
             small_dft<R2, -1>(v, [&](int k2, double2 X) {
                 const int k = kCrt<R1, R2>.k[k1][k2];
-                if (k < G::H) out[(size_t)k * MM] = X;
+                if (k < G::H) put(k, X);
                 else
-                    out[(size_t)(P - k) * MM] = make_double2(X.x, -X.y);
+                    put(P - k, make_double2(X.x, -X.y));
             });
         }
     }
@@ -397,15 +413,15 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __r
 // ---------------------------------------------------------------------------
 template<int N, class T>
 __global__ __launch_bounds__(Par<N>::T) __attribute__((amdgpu_waves_per_eu(5))) void k_parent_fwd_plane(
-    const double2* __restrict__ mid, typename Spec<T>::C* __restrict__ spec, int rows)
+    const double2* __restrict__ mid, typename Spec<T>::C* __restrict__ spec, int rows, Slice sl)
 {
     using G = Par<N>;
     constexpr int      M = G::M, P = G::P, R1 = G::R1, R2 = G::R2, PS = G::PS;
     __shared__ double2 in[M * M];   // [y][x]
     __shared__ double2 Y[M * PS];   // [x][qy]
     __shared__ double2 tab[R1];
-    const int          l = threadIdx.x, kz = blockIdx.x / rows, row = blockIdx.x - kz * rows;
-    mid += ((size_t)row * G::H + kz) * (M * M);
+    const int          l = threadIdx.x, zl = blockIdx.x / rows, row = blockIdx.x - zl * rows, kz = sl.z0 + zl;
+    mid += ((size_t)row * sl.nz + zl) * (M * M);
     root_table<R1>(tab);
     for (int q = l; q < M * M; q += G::T) in[q] = mid[q];
     __syncthreads();
@@ -424,7 +440,7 @@ __global__ __launch_bounds__(Par<N>::T) __attribute__((amdgpu_waves_per_eu(5))) 
         leg_roots<R1, -1>(k1, tab, w);
         forward_first<N>(w, v, [&](int n) { return Y[n * PS + qy]; });
         small_dft<R2, -1>(v, [&](int k2, double2 X) {
-            spec[spec_at(kz * G::PP + (k2 * R1 + k1) * P + qy, row, rows)] = Spec<T>::put(X);
+            spec[spec_at(kz * G::PP + (k2 * R1 + k1) * P + qy, sl.chunk0, row, rows)] = Spec<T>::put(X);
         });
     }
 }
@@ -470,17 +486,17 @@ __device__ inline void mac_entries(const int2* __restrict__ ent, int& e, int end
 template<class T>
 __global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int4* __restrict__ group,
     const int* __restrict__ begin, const int2* __restrict__ ent, int ngroup, int ntgt, int nsrc, int ncomp, const double2* __restrict__ ghat,
-    const typename Spec<T>::C* __restrict__ sspec, typename Spec<T>::C* __restrict__ tspec, int nchunk, int nseg)
+    const typename Spec<T>::C* __restrict__ sspec, typename Spec<T>::C* __restrict__ tspec, Slice sl, int nseg)
 {
     __shared__ double2 Gs[(kParentNone + 1) * 64];
     const int          r = blockIdx.x >> 3, chunk = (r / nseg) * 8 + (blockIdx.x & 7), seg = r % nseg;
-    if (chunk >= nchunk) return;  // the whole workgroup
+    if (chunk >= sl.nchunk) return;  // the whole workgroup
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (wave == kMacWaves - 1) Gs[kParentNone * 64 + lane] = make_double2(0.0, 0.0);
     for (int o = wave; o < 27; o += kMacWaves)
     {
         // stored: offsets 13 (own parent) to 26; offset o < 13 is the opposite of 26 - o
-        double2 g = ghat[((size_t)chunk * 14 + (o < 13 ? 13 - o : o - 13)) * 64 + lane];
+        double2 g = ghat[((size_t)(sl.chunk0 + chunk) * 14 + (o < 13 ? 13 - o : o - 13)) * 64 + lane];
         if (o < 13) g.y = -g.y;
         Gs[o * 64 + lane] = g;
     }
@@ -528,20 +544,20 @@ __device__ inline int window(int a, int b)  // window point of (a, b), W or more
 
 template<int N, class T>
 __global__ __launch_bounds__(Par<N>::T) void k_parent_inv_plane(
-    const typename Spec<T>::C* __restrict__ spec, double2* __restrict__ mid, int rows)
+    const typename Spec<T>::C* __restrict__ spec, double2* __restrict__ mid, int rows, Slice sl)
 {
     using G = Par<N>;
     constexpr int      P = G::P, R1 = G::R1, R2 = G::R2, W = G::W, WS = G::WS;
     static_assert(P * WS <= G::PP, "the x leg's outputs take the place of its inputs");
     __shared__ double2 buf[G::PP];  // [k2][a][qy], then [qy][x]
-    const int          l = threadIdx.x, kz = blockIdx.x / rows, row = blockIdx.x - kz * rows;
+    const int          l = threadIdx.x, zl = blockIdx.x / rows, row = blockIdx.x - zl * rows, kz = sl.z0 + zl;
     mid += ((size_t)row * G::H + kz) * (W * W);
     double2 u[R1], v[R2];
     for (int it = l; it < R2 * P; it += G::T)
     {
         const int k2 = it / P, at = k2 * (R1 * P) + it - k2 * P;
 #pragma unroll
-        for (int k = 0; k < R1; ++k) u[k] = Spec<T>::get(spec[spec_at(kz * G::PP + at + k * P, row, rows)]);
+        for (int k = 0; k < R1; ++k) u[k] = Spec<T>::get(spec[spec_at(kz * G::PP + at + k * P, sl.chunk0, row, rows)]);
         inverse_first<R1>(u);
 #pragma unroll
         for (int k = 0; k < R1; ++k) buf[at + k * P] = u[k];
@@ -719,40 +735,100 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_ghat_leg(
     }
     if (AXIS < 2) out[(long)o * G::NF + f] = s;
     else
-        out[spec_at(kz * G::PP + lo * P + hi, o, 14)] = s;
+        out[spec_at(kz * G::PP + lo * P + hi, 0, o, 14)] = s;
 }
 
 // ---------------------------------------------------------------------------
 // Launches
 // ---------------------------------------------------------------------------
 inline unsigned blocks_of(long total, int per) { return (unsigned)((total + per - 1) / per); }
+constexpr size_t round256(size_t b) { return (b + 255) / 256 * 256; }
+
+// Where a pass keeps its spectra and columns, for ns source and nt target
+// parents (times components) and values of `elem` bytes, in bytes from the
+// start of its scratch.  All planes in one round: the columns of the forward
+// legs lie where the target spectra come later, those of the inverse legs
+// where the source spectra were.  In rounds of nz planes: the inverse legs'
+// columns apart, since the last leg needs all planes; the forward z leg runs
+// again every round.
+template<class G>
+struct Layout
+{
+    int    nz = 0;  // planes a round; 0: does not fit
+    size_t mid_s = 0, mid_t = 0, sspec = 0, tspec = 0, bytes = 0;
+
+    static Slice slice(int z0, int nz)
+    {
+        nz = std::min(nz, G::H - z0);
+        const int c0 = z0 * G::PP / 64;
+        return Slice{z0, nz, c0, ((z0 + nz) * G::PP + 63) / 64 - c0};
+    }
+    Layout(long ns, long nt, size_t elem, int planes) : nz(planes)
+    {
+        size_t chunks = 0;
+        for (int z0 = 0; z0 < G::H; z0 += nz) chunks = std::max<size_t>(chunks, slice(z0, nz).nchunk);
+        const size_t S = round256(ns * chunks * 64 * elem), T = round256(nt * chunks * 64 * elem);
+        const size_t ms = round256((size_t)ns * nz * G::M * G::M * sizeof(double2));
+        const size_t mt = round256((size_t)nt * G::H * G::W * G::W * sizeof(double2));
+        sspec = nz == G::H ? 0 : mt;
+        tspec = mid_s = nz == G::H ? std::max(S, mt) : mt + S;
+        bytes = tspec + std::max(T, ms);
+    }
+    static Layout fit(long ns, long nt, size_t elem, size_t room)
+    {
+        Layout l(ns, nt, elem, G::H);
+        for (int z = 2; l.bytes > room && z <= G::H; ++z)  // z rounds
+            if ((G::H + z - 1) / z < l.nz) l = Layout(ns, nt, elem, (G::H + z - 1) / z);
+        if (l.bytes > room) l.nz = 0;
+        return l;
+    }
+};
 
 template<int N>
 struct Run
 {
     using G = Par<N>;
+    using L = Layout<G>;
     template<class T>
     static void pass(hipStream_t s, const ParentPass& p, const double* src, double* dst, double scale, const Batch& b)
     {
         using C = typename Spec<T>::C;
         const long ns = (long)p.nsrc * b.k, nt = (long)p.ntgt * b.k;
-        hipLaunchKernelGGL(k_parent_fwd_z<N>, dim3(blocks_of(ns * G::M * G::M, kLineThreads)), dim3(kLineThreads), 0, s,
-            src, b.fstride, p.src_child, p.nsrc, b.k, p.mid);
-        hipLaunchKernelGGL((k_parent_fwd_plane<N, T>), dim3((unsigned)(ns * G::H)), dim3(G::T), 0, s, p.mid, (C*)p.sspec,
-            (int)ns);
+        const L    l = L::fit(ns, nt, sizeof(C), p.bytes);
+        if (l.nz == 0) throw std::logic_error("parent_pass: scratch too small");
+        char*    at = static_cast<char*>(p.scratch);
+        double2 *mid_s = reinterpret_cast<double2*>(at + l.mid_s), *mid_t = reinterpret_cast<double2*>(at + l.mid_t);
+        C *      sspec = reinterpret_cast<C*>(at + l.sspec), *tspec = reinterpret_cast<C*>(at + l.tspec);
         // (group, component) pairs a wave: fewer read the kernel values more often, more leave a chunk's
         // sources to L2 for longer (4290 blocks, 2 and 4 pairs: FP64 1.058 and 1.065 ms, with fewer blocks
         // 0.389 and 0.404; FP32, three components, 1.95 and 1.83)
         constexpr int kRun = sizeof(T) == 8 ? 2 : 4;
-        const int nchunk = G::NCH, nseg = (int)std::min(64L, ((long)p.ngroup * b.k + kRun * kMacWaves - 1) / (kRun * kMacWaves));
-        hipLaunchKernelGGL(k_parent_mac<T>, dim3((unsigned)((nchunk + 7) / 8 * 8 * nseg)), dim3(64 * kMacWaves), 0, s,
-            p.group, p.begin, p.entries, p.ngroup, p.ntgt, p.nsrc, b.k, p.ghat, (const C*)p.sspec, (C*)p.tspec, nchunk, nseg);
-        hipLaunchKernelGGL(
-            (k_parent_inv_plane<N, T>), dim3((unsigned)(nt * G::H)), dim3(G::T), 0, s, (const C*)p.tspec, p.mid,
-            (int)nt);
+        const int nseg = (int)std::min(64L, ((long)p.ngroup * b.k + kRun * kMacWaves - 1) / (kRun * kMacWaves));
+        const dim3 zgrid(blocks_of(ns * G::M * G::M, kLineThreads)), zthreads(kLineThreads);
+        for (int z0 = 0; z0 < G::H; z0 += l.nz)
+        {
+            const Slice sl = L::slice(z0, l.nz);
+            if (l.nz == G::H)
+                hipLaunchKernelGGL((k_parent_fwd_z<N, false>), zgrid, zthreads, 0, s, src, b.fstride, p.src_child, p.nsrc,
+                    b.k, mid_s, 0, G::H);
+            else
+                hipLaunchKernelGGL((k_parent_fwd_z<N, true>), zgrid, zthreads, 0, s, src, b.fstride, p.src_child, p.nsrc,
+                    b.k, mid_s, sl.z0, sl.nz);
+            hipLaunchKernelGGL((k_parent_fwd_plane<N, T>), dim3((unsigned)(ns * sl.nz)), dim3(G::T), 0, s, mid_s, sspec,
+                (int)ns, sl);
+            hipLaunchKernelGGL(k_parent_mac<T>, dim3((unsigned)((sl.nchunk + 7) / 8 * 8 * nseg)), dim3(64 * kMacWaves), 0,
+                s, p.group, p.begin, p.entries, p.ngroup, p.ntgt, p.nsrc, b.k, p.ghat, sspec, tspec, sl, nseg);
+            hipLaunchKernelGGL(
+                (k_parent_inv_plane<N, T>), dim3((unsigned)(nt * sl.nz)), dim3(G::T), 0, s, tspec, mid_t, (int)nt, sl);
+        }
         hipLaunchKernelGGL(k_parent_inv_z<N>, dim3(blocks_of(nt * 4 * G::NN, kLineThreads)), dim3(kLineThreads), 0, s,
-            p.mid, p.tgt_child, p.ntgt, b.k, dst, b.fstride,
+            mid_t, p.tgt_child, p.ntgt, b.k, dst, b.fstride,
             scale / ((double)G::P * G::P * G::P));
+    }
+    static size_t bytes(long ns, long nt, size_t elem, size_t room)
+    {
+        const L l = room ? L::fit(ns, nt, elem, room) : L(ns, nt, elem, G::H);
+        return l.nz ? l.bytes : 0;
     }
     static void spectra(hipStream_t s, const double* sample, double2* a, double2* b, double2* ghat)
     {
@@ -799,6 +875,11 @@ void parent_pass(hipStream_t s, int n, int prec, const ParentPass& p, const doub
         else
             R::template pass<float>(s, p, src, dst, scale, b);
     });
+}
+size_t parent_bytes(int n, int prec, long nsrc, long ntgt, size_t room)
+{
+    const size_t elem = prec == 0 ? sizeof(double2) : sizeof(float2);
+    return on_n(n, [&](auto r) { return decltype(r)::bytes(nsrc, ntgt, elem, room); });
 }
 void parent_spectra(hipStream_t s, int n, const double* sample, double2* a, double2* b, double2* ghat)
 {

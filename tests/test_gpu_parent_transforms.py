@@ -6,6 +6,7 @@ side leave errors of a few 1e-15 of the largest contribution to a target: 1e-12
 relative to the whole field.  FP32 spectra carry 6e-8 a value: 1e-6."""
 import numpy as np
 import pytest
+import torch
 
 from iblgf_amd import FLAG_LEAF, PREC_FP16X3_FORWARD, PREC_FP64, PREC_MIXED, PoissonSolver, Tree, lib, setups
 
@@ -60,6 +61,66 @@ def test_adaptive_tree_two_components(oracle_mod, extent, precision):
     v = setups.VortexRings(seed=7, block_extent=extent, base_blocks=4, nref=2, nrings=3, centre_range=4.0,
                            radius=(4.0, 8.0), core=(1.5, 2.5), refinement_factor=0.5)
     _check(oracle_mod, v.tree, 2, precision, 1e-12 if precision == PREC_FP64 else 1e-6)
+
+
+def _solver(tree, precision, ncomp):
+    s = PoissonSolver(tree)
+    s.set_precision(precision)
+    rng = np.random.default_rng(12)
+    src, dst = [s.field() for _ in range(ncomp)], [s.field() for _ in range(ncomp)]
+    for f in src:
+        s.upload(f, rng.standard_normal(s.shape))
+    return s, src, dst
+
+
+@pytest.mark.parametrize("extent", [6, 8, 10, 14, 16])
+@pytest.mark.parametrize("region", [(1, 1, 1), (2, 3, 1), (4, 3, 3), None])
+def test_scratch_in_rounds(extent, region):
+    """The spectra of whole parents in the memory that block spectra leave: at
+    once, in rounds of some frequencies (FP64 solves of as many components as
+    the work arrays hold, here, on every mesh but the one of a single block),
+    and, for a single block, outside it.  Frequencies are independent, so the
+    results are equal bit for bit."""
+    print(f"case: scratch of whole parents, {extent}^3 blocks, region {region}", flush=True)
+    if region:
+        t = _uniform(extent, region)
+    else:
+        t = setups.VortexRings(seed=7, block_extent=extent, base_blocks=4, nref=1, nrings=1, centre_range=2.0,
+                               radius=(3.0, 4.0), core=(1.5, 2.0), refinement_factor=0.3).tree
+    s, src, dst = _solver(t, PREC_FP64, 3)
+    for f, d in zip(src, dst):
+        s.apply_lgf(f, d)  # one component in work arrays of one
+    one = [s.download(d) for d in dst]
+    s.apply_lgf_batch(src, dst)  # three in arrays of three
+    assert all(np.array_equal(s.download(d), x) for d, x in zip(dst, one))
+    s.apply_lgf(src[0], dst[0])  # one in arrays of three: at once
+    assert np.array_equal(s.download(dst[0]), one[0])
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
+def test_memory_of_a_component(precision):
+    """A solve takes the memory of its work arrays, four fields and two
+    block spectra of FP64 a component, and nothing beside them however its
+    parents lie.  (Allocations come in whole pages of 2 MiB.)"""
+    print(f"case: memory a component, precision {precision}", flush=True)
+    t = setups.VortexRings(seed=7, block_extent=16, base_blocks=4, nref=2, nrings=3, centre_range=4.0,
+                           radius=(4.0, 8.0), core=(1.5, 2.5), refinement_factor=0.5).tree
+    s, src, dst = _solver(t, precision, 6)
+    s.prepare()
+    s.apply_lgf(src[0], dst[0])
+    n, nb = t.n, s.shape[0]
+    P = 2 * n - 1
+    per = nb * (4 * n**3 * 8 + 2 * P * P * (P // 2 + 1) * 16)
+
+    def used(k):
+        s.apply_lgf_batch(src[:k], dst[:k])
+        s.sync()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    at = [used(k) for k in (1, 3, 6)]
+    assert at[1] - at[0] <= 2 * per + (16 << 20)
+    assert at[2] - at[0] <= 5 * per + (16 << 20)
 
 
 def test_wrapped_keys_keep_the_block_path(oracle_mod):

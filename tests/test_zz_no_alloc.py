@@ -2,13 +2,15 @@
 ABI: its results equal iblgf_gpu_apply_lgf's bit for bit (same kernels, same
 order, only the work memory differs) on two calls in a row, the second on a
 smaller tree, for the Laplace and integrating-factor kernels and in mixed
-precision; it refuses unprepared solves (IBLGF_ERR_STATE) and trees whose work
+precision; whatever other solves of the context have run in between, it
+allocates and frees nothing, and a graph captured around it stays valid; it refuses unprepared solves (IBLGF_ERR_STATE) and trees whose work
 exceeds the fixed scratch (IBLGF_ERR_UNSUPPORTED)."""
 import numpy as np
 import pytest
+import torch
 
-from iblgf_amd import (IBLGF_ERR_STATE, IBLGF_ERR_UNSUPPORTED, KERNEL_IF, KERNEL_LAPLACE, PREC_MIXED, IblgfError,
-                       PoissonSolver, setups)
+from iblgf_amd import (IBLGF_ERR_STATE, IBLGF_ERR_UNSUPPORTED, KERNEL_IF, KERNEL_LAPLACE, PREC_FP64, PREC_MIXED,
+                       IblgfError, PoissonSolver, Tree, setups)
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +79,66 @@ def test_noalloc_mixed_precision_and_size_limit():
     solver.set_precision(PREC_MIXED)
     a, b = _both(solver, src)
     _equal_where_written(a, b, KERNEL_LAPLACE, wl.arrays["flags"])
+
+
+def _block():
+    """One block of 6^3 cells: its whole parents do not fit the region beside the coarse levels' spectra."""
+    t = Tree((-24,) * 3, (48,) * 3, 6, 1.0 / 6, [(0, 0, 0, 6, 6, 6)])
+    return t.init_refine(0).build_masks()
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("tree", ["rings", "uniform", "block"])
+def test_other_solves_between(tree, precision):
+    print(f"case: noalloc between other solves, {tree}, precision {precision}", flush=True)
+    t = {"rings": lambda: _rings(6).tree, "uniform": lambda: setups.UniformGaussians(seed=1000).tree,
+         "block": _block}[tree]()
+    rng = np.random.default_rng(4)
+    src = rng.standard_normal((t.info()["nblocks"],) + (t.n,) * 3)
+    ref_solver = PoissonSolver(t)
+    ref_solver.set_precision(precision)
+    f, g = ref_solver.field(), ref_solver.field()
+    ref_solver.upload(f, src)
+    ref_solver.apply_lgf(f, g)
+    ref = ref_solver.download(g)
+
+    s = PoissonSolver(t)
+    s.set_precision(precision)
+    fi, fo = [s.field() for _ in range(6)], [s.field() for _ in range(6)]
+    out = s.field()
+    for x in fi:
+        s.upload(x, src)
+    s.prepare()
+
+    def check():
+        s.upload(out, np.zeros_like(src))
+        before = _free()
+        s.apply_lgf_noalloc(fi[0], out)
+        assert _free() == before
+        assert np.array_equal(s.download(out), ref)
+
+    s.apply_lgf_batch(fi[:3], fo[:3], kernel=KERNEL_IF, alpha_base=0.4)  # grows the work arrays only
+    check()
+    # captured by the caller, then replayed after solves that grow what the context keeps
+    st = torch.cuda.ExternalStream(s.stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(st):
+        graph.capture_begin(capture_error_mode="thread_local")
+        s.apply_lgf_noalloc(fi[0], out)
+        graph.capture_end()
+    s.apply_lgf_batch(fi[:3], fo[:3])
+    check()
+    s.apply_lgf_batch(fi, fo)
+    check()
+    for _ in range(3):
+        s.upload(out, np.zeros_like(src))
+        with torch.cuda.stream(st):
+            graph.replay()
+        s.sync()
+        assert np.array_equal(s.download(out), ref)
+        s.apply_lgf(fi[1], fo[1])  # eager work between replays
