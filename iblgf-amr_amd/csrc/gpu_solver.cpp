@@ -922,7 +922,13 @@ void GpuSolver::build_pass(PassPlan& p, int L, int idx, bool nbonly)
         if (fwd[i] >= lvl_begin_[L + 1]) throw std::logic_error("pass plan: sources finer than the pass level");
     p.inv.upload(inv);
     for (const std::vector<int>* l : {&fwd, &inv})
-        for (int slot : *l) p.spec_slots = std::max(p.spec_slots, slot + 1);
+        for (int slot : *l)
+        {
+            p.spec_slots = std::max(p.spec_slots, slot + 1);
+            if (slot < lvl_begin_[base_level_]) p.top_slots = std::max(p.top_slots, slot + 1);
+        }
+    while (p.nfwd_top < static_cast<int>(fwd.size()) && fwd[p.nfwd_top] < p.top_slots) ++p.nfwd_top;
+    for (int slot : inv) p.ninv_base += slot >= p.top_slots ? 1 : 0;
     p.ninv_top = 0;
     while (p.ninv_top < static_cast<int>(inv.size()) && inv[p.ninv_top] >= lvl_begin_[L] &&
            inv[p.ninv_top] < lvl_begin_[L + 1])
@@ -1086,10 +1092,12 @@ const double* GpuSolver::if_iv(double alpha)
     return (if_iv_[alpha] = std::move(a)).p;
 }
 
-const void* GpuSolver::ghat(bool laplace, int d, double alpha)
+int GpuSolver::mac_precision(const MacLevelPlan& m) const { return m.lambda < base_level_ ? kPrecFp64 : precision_; }
+
+const void* GpuSolver::ghat(bool laplace, int d, double alpha, int prec)
 {
     double2* g64 = laplace ? ghat_laplace(d) : ghat_if(alpha);
-    if (precision_ == 0) return g64;
+    if (prec == kPrecFp64) return g64;
     DevArray<float2>* slot = nullptr;
     if (laplace)
     {
@@ -1125,14 +1133,14 @@ void GpuSolver::prepare_laplace(int k)
         {
             PassPlan& p = pass(l, nl, false);
             prepare_pass(p);
-            reserve_parents(p, k);
+            reserve_extra(p, k);
         }
     // What an allocation-free solve needs beyond its region: of a size that
     // holds in every precision, and kept while the tree is loaded.
     size_t one = 0;
     for (const auto& kv : passes_)
-        if (kv.second->npar_tgt > 0 && amr2amr(*kv.second) && !fits_region(*kv.second))
-            one = std::max(one, launch::parent_bytes(n_, kPrecFp64, kv.second->npar_src, kv.second->npar_tgt, 0));
+        for (int prec : {kPrecFp64, kPrecMixed})
+            if (amr2amr(*kv.second)) one = std::max(one, region_spectra(*kv.second, prec).extra_bytes);
     if (par_one_.n == 0 && one > 0 && region_bytes(kPrecMixed) <= kNoallocScratchBytes)
         par_one_.alloc(one / sizeof(double2));
     sync();
@@ -1140,7 +1148,7 @@ void GpuSolver::prepare_laplace(int k)
 
 void GpuSolver::prepare_pass(PassPlan& p)
 {
-    for (auto& m : p.mac) ghat(true, m.d, 0.0);
+    for (auto& m : p.mac) ghat(true, m.d, 0.0, mac_precision(m));
     if (p.npar_tgt > 0) parent_ghat();
 }
 
@@ -1164,76 +1172,96 @@ const double2* GpuSolver::parent_ghat()
     return par_ghat_.p;
 }
 
-// What the block spectra of a pass (slots below spec_slots: coarser levels,
-// and level-L blocks that are not part of whole parents) leave of the spectra's
-// memory, `spec` of `bytes`, when they lie at its start: the whole parents' scratch.
-GpuSolver::SpecPtrs GpuSolver::spectra(const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes) const
+// The spectra of one pass in the memory `spec` of `bytes`: the block spectra
+// (of the coarser levels, and of level-L blocks that are not part of whole
+// parents), component by component without gaps for other slots, and what is
+// left for the whole parents.  What does not fit, even with the parents in
+// rounds (few and partly filled parents), goes to `extra`, of which it
+// takes extra_bytes.
+//
+// With FP32 spectra those below the base level are FP64 all the same: few
+// blocks, but the ones whose rounding reaches farthest.  In a 4290-block solve of
+// three components with FP32 spectra, 64 blocks of one level gave most of the
+// error: 9.1e-8, 5.2e-8, 1.6e-7 against FP64, 3.5e-8, 6.5e-8, 5.1e-8 with
+// theirs in FP64, for 0.24 of 9.74 ms.
+GpuSolver::SpecPtrs GpuSolver::spectra(
+    const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes, void* extra) const
 {
-    const size_t elem = prec == kPrecFp64 ? sizeof(double2) : sizeof(float2);
-    const size_t half = p.npar_tgt > 0 ? round256(static_cast<size_t>(p.spec_slots) * nf_ * b.k * elem) : bytes / 2;
-    char*        at = static_cast<char*>(spec);
-    SpecPtrs     s{at, at + half, at + 2 * half, bytes - 2 * half, b};
-    if (p.npar_tgt > 0) s.b.sstride = static_cast<long>(p.spec_slots) * nf_;
+    const bool   fp32 = prec != kPrecFp64;
+    const int    ntop = fp32 ? p.top_slots : 0;
+    const size_t elem = fp32 ? sizeof(float2) : sizeof(double2), nf = nf_, k = b.k;
+    const size_t top = round256(ntop * nf * k * sizeof(double2)), half = round256((p.spec_slots - ntop) * nf * k * elem);
+    uintptr_t    at = reinterpret_cast<uintptr_t>(spec), ex = reinterpret_cast<uintptr_t>(extra);
+    auto         ptr = [](uintptr_t a) { return reinterpret_cast<void*>(a); };
+    SpecPtrs     s;
+    s.b = s.btop = b;
+    s.b.sstride = static_cast<long>((p.spec_slots - ntop) * nf);
+    s.btop.sstride = static_cast<long>(ntop * nf);
+    if (2 * (top + half) > bytes)
+    {
+        s.stop = ptr(ex);
+        s.ttop = ptr(ex + top);
+        s.extra_bytes = 2 * top;
+    }
+    else
+    {
+        s.stop = ptr(at);
+        s.ttop = ptr(at + top);
+        at += 2 * top;
+        bytes -= 2 * top;
+    }
+    s.sspec = ptr(at - ntop * nf * elem);  // slots are counted from 0
+    s.tspec = ptr(at + half - ntop * nf * elem);
+    s.rest = ptr(at + 2 * half);
+    s.rest_bytes = bytes - 2 * half;
+    if (p.npar_tgt > 0)
+    {
+        const long ns = static_cast<long>(p.npar_src) * b.k, nt = static_cast<long>(p.npar_tgt) * b.k;
+        if (s.rest_bytes == 0 || launch::parent_bytes(n_, prec, ns, nt, s.rest_bytes) == 0)
+        {
+            s.rest = ptr(ex + s.extra_bytes);
+            s.rest_bytes = launch::parent_bytes(n_, prec, ns, nt, 0);
+            s.extra_bytes += s.rest_bytes;
+        }
+    }
     return s;
 }
 
-static bool parents_fit(int n, int prec, const PassPlan& p, int k, size_t room)
+// As an allocation-free solve has them in its region (sizes only).
+GpuSolver::SpecPtrs GpuSolver::region_spectra(const PassPlan& p, int prec) const
 {
-    return room > 0 && launch::parent_bytes(n, prec, static_cast<long>(p.npar_src) * k,
-                           static_cast<long>(p.npar_tgt) * k, room) > 0;
-}
-
-// Whether the whole parents of a pass fit the region of an allocation-free
-// solve in every precision.
-bool GpuSolver::fits_region(const PassPlan& p) const
-{
-    for (int prec : {kPrecFp64, kPrecMixed})
-    {
-        const size_t sb = spec_region_bytes(prec);
-        if (!parents_fit(n_, prec, p, 1, spectra(p, prec, batch(1), nullptr, 2 * sb).rest_bytes)) return false;
-    }
-    return true;
+    return spectra(p, prec, batch(1), nullptr, 2 * spec_region_bytes(prec), nullptr);
 }
 
 // The passes of the AMR2AMR solves.
 bool GpuSolver::amr2amr(const PassPlan& p) const { return !p.neighbor_only && p.idx >= 15 && p.idx < 30; }
 
-// Scratch of a pass of k components whose whole parents do not fit beside its
-// block spectra even in rounds (few and partly filled parents), for all of
-// their frequencies at once.
-void GpuSolver::reserve_parents(const PassPlan& p, int k)
+// Memory beside the work arrays for a pass of k components.
+void GpuSolver::reserve_extra(const PassPlan& p, int k)
 {
-    if (p.npar_tgt == 0) return;
     const size_t bytes = 2 * round256(static_cast<size_t>(nb_) * nf_ * std::max(k, work_.k) * sizeof(double2));
-    if (parents_fit(n_, precision_, p, k, spectra(p, precision_, batch(k), nullptr, bytes).rest_bytes)) return;
-    const size_t need = launch::parent_bytes(
-        n_, precision_, static_cast<long>(p.npar_src) * k, static_cast<long>(p.npar_tgt) * k, 0);
+    const size_t need = spectra(p, precision_, batch(k), nullptr, bytes, nullptr).extra_bytes;
     if (par_extra_.n * sizeof(double2) >= need) return;
     sync();         // passes in flight still use the old array
     drop_graphs();  // captured graphs point at it
     par_extra_.alloc(need / sizeof(double2));
 }
 
+// The spectra of a pass about to run.  In a region nothing is used but the
+// region, the plans and what prepare has put aside.
+GpuSolver::SpecPtrs GpuSolver::pass_spectra(const PassPlan& p, const Batch& b)
+{
+    if (!wp_.region) reserve_extra(p, b.k);
+    const DevArray<double2>& extra = wp_.region ? par_one_ : par_extra_;
+    const SpecPtrs           s = spectra(p, precision_, b, wp_.spec, wp_.spec_bytes, extra.p);
+    if (s.extra_bytes > extra.n * sizeof(double2)) throw std::logic_error("pass: spectra do not fit their memory");
+    return s;
+}
+
 void GpuSolver::run_parents(PassPlan& p, double scale, const SpecPtrs& sp)
 {
-    ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_group.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt,
+    const ParentPass pp{p.par_src.p, p.par_tgt.p, p.par_group.p, p.par_begin.p, p.par_ent.p, p.npar_src, p.npar_tgt,
         static_cast<int>(p.par_group.n), parent_ghat(), sp.rest, sp.rest_bytes};
-    if (wp_.region)
-    {
-        // nothing but the region, the plans and what prepare has put aside
-        if (!fits_region(p))
-        {
-            if (!par_one_.p) throw std::logic_error("whole parents: no scratch beside the region");
-            pp.scratch = par_one_.p;
-            pp.bytes = par_one_.n * sizeof(double2);
-        }
-    }
-    else if (!parents_fit(n_, precision_, p, sp.b.k, sp.rest_bytes))
-    {
-        reserve_parents(p, sp.b.k);
-        pp.scratch = par_extra_.p;
-        pp.bytes = par_extra_.n * sizeof(double2);
-    }
     launch::parent_pass(stream_, n_, precision_, pp, wp_.src, wp_.tgt, scale, sp.b);
 }
 
@@ -1244,7 +1272,7 @@ void GpuSolver::prepare_if(double alpha_base)
         const double alpha = alpha_base * std::pow(4.0, l - base_level_);
         if_iv(alpha);
         for (int nl = 0; nl < 2; ++nl)
-            if (!pass(l, nl, true).mac.empty()) ghat(false, 0, alpha);
+            if (!pass(l, nl, true).mac.empty()) ghat(false, 0, alpha, precision_);
     }
     sync();
 }
@@ -1256,7 +1284,7 @@ int GpuSolver::inverse_legs() const { return precision_ == kPrecF16x3Forward ? k
 
 void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, const Batch& batch)
 {
-    const SpecPtrs sp = spectra(p, precision_, batch, wp_.spec, wp_.spec_bytes);
+    const SpecPtrs sp = pass_spectra(p, batch);
     const Batch&   b = sp.b;
     double*      fmm_s = wp_.fmm_s;
     double*      fmm_t = wp_.fmm_t;
@@ -1264,13 +1292,13 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
     const double P = 2.0 * n_ - 1.0, iscale = scale / (P * P * P);
     // Kernel spectra first: building one launches work on the solver stream.
     std::vector<const void*> gh(p.mac.size());
-    for (size_t i = 0; i < p.mac.size(); ++i) gh[i] = ghat(laplace, p.mac[i].d, alpha);
+    for (size_t i = 0; i < p.mac.size(); ++i) gh[i] = ghat(laplace, p.mac[i].d, alpha, mac_precision(p.mac[i]));
     if (p.sep_t.size() > 0)
     {
         const double* iv = if_iv(alpha);
         timer_.begin(stream_);
         launch::if_separable(stream_, n_, wp_.src, static_cast<double*>(wp_.spec), wp_.tgt, p.sep_z.p,
-            p.sep_z.size() / 3, p.sep_t.p, p.sep_t.size() / 10, iv, b, b.sstride);
+            p.sep_z.size() / 3, p.sep_t.p, p.sep_t.size() / 10, iv, batch, batch.sstride);
         timer_.end(stream_, KC_OTHER, 0);
     }
     if (p.neighbor_only && p.mac.empty()) return;
@@ -1313,19 +1341,24 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
         timer_.end(A, KC_MAC, p.par_npairs * b.k);
     }
     const int nfine = static_cast<int>(p.fwd.size()) - p.nfwd_coarse;
+    const auto top_spectra = [&](void* spec, int count) {  // blocks below the base level
+        return precision_ == kPrecFp64 ? TopSpectra{} : TopSpectra{static_cast<double2*>(spec), sp.btop.sstride, count};
+    };
     timer_.begin(A);
     launch::forward_dft(A, n_, forward_legs(), fmm_s, p.fwd.p + p.nfwd_coarse, nfine, sp.sspec, b, wp_.src, 0);
     timer_.end(A, KC_FORWARD, static_cast<long>(nfine) * b.k);
     timer_.begin(B);
-    launch::forward_dft(B, n_, forward_legs(), fmm_s, p.fwd.p, p.nfwd_coarse, sp.sspec, b);
+    launch::forward_dft(B, n_, forward_legs(), fmm_s, p.fwd.p, p.nfwd_coarse, sp.sspec, b, nullptr, -1,
+        top_spectra(sp.stop, p.nfwd_top));
     timer_.end(B, KC_FORWARD, static_cast<long>(p.nfwd_coarse) * b.k);
     for (size_t i = 0; i < p.mac.size(); ++i)
     {
         const MacLevelPlan& m = p.mac[i];
         hipStream_t         s = m.lambda == L ? A : B;
         timer_.begin(s);
-        launch::spectral_mac(s, n_, precision_, m.groups.p, m.groups.size(), m.srcs.p, m.rowoff.p, m.olist.p,
-            m.nused, m.compact, gh[i], sp.sspec, sp.tspec, b, m.queue.p);
+        const bool low = precision_ != kPrecFp64 && m.lambda < base_level_;
+        launch::spectral_mac(s, n_, mac_precision(m), m.groups.p, m.groups.size(), m.srcs.p, m.rowoff.p, m.olist.p,
+            m.nused, m.compact, gh[i], low ? sp.stop : sp.sspec, low ? sp.ttop : sp.tspec, low ? sp.btop : b, m.queue.p);
         timer_.end(s, KC_MAC, m.npairs * b.k);
     }
     // Level-L targets (first in inv) add into the target array, coarser ones
@@ -1335,7 +1368,8 @@ void GpuSolver::run_pass(PassPlan& p, double scale, bool laplace, double alpha, 
     launch::inverse_dft(A, n_, inverse_legs(), sp.tspec, p.inv.p, ntop, wp_.tgt, iscale, true, b);
     timer_.end(A, KC_INVERSE, static_cast<long>(ntop) * b.k);
     timer_.begin(B);
-    launch::inverse_dft(B, n_, inverse_legs(), sp.tspec, p.inv.p + ntop, nrest, fmm_t, iscale, false, b);
+    launch::inverse_dft(B, n_, inverse_legs(), sp.tspec, p.inv.p + ntop, nrest, fmm_t, iscale, false, b,
+        top_spectra(sp.ttop, static_cast<int>(p.inv.size()) - p.ninv_base));
     timer_.end(B, KC_INVERSE, static_cast<long>(nrest) * b.k);
     if (coarse)
     {
@@ -1678,9 +1712,9 @@ void GpuSolver::apply_if_batch(const int* src, const int* dst, int k, double alp
     mesh_ = kMeshCell;
 }
 
-bool GpuSolver::has_ghat(bool laplace, int d, double alpha) const
+bool GpuSolver::has_ghat(bool laplace, int d, double alpha, int prec) const
 {
-    if (precision_ == 0) return laplace ? ghat_lap_.count(d) > 0 : ghat_if_.count(alpha) > 0;
+    if (prec == kPrecFp64) return laplace ? ghat_lap_.count(d) > 0 : ghat_if_.count(alpha) > 0;
     return laplace ? ghat_lap32_.count(d) > 0 : ghat_if32_.count(alpha) > 0;
 }
 
@@ -1695,9 +1729,9 @@ bool GpuSolver::prepared(bool laplace, double alpha_base) const
             const auto it = passes_.find(pass_key(l, fmm_mask_idx_gen(MASK_AMR2AMR, l - base_level_, nl), !laplace));
             if (it == passes_.end() || (!laplace && !if_iv_.count(alpha))) return false;
             for (const auto& m : it->second->mac)
-                if (!has_ghat(laplace, m.d, alpha)) return false;
-            if (it->second->npar_tgt > 0 && (par_ghat_.n == 0 || (par_one_.n == 0 && !fits_region(*it->second))))
-                return false;
+                if (!has_ghat(laplace, m.d, alpha, mac_precision(m))) return false;
+            if (it->second->npar_tgt > 0 && par_ghat_.n == 0) return false;
+            if (region_spectra(*it->second, precision_).extra_bytes > par_one_.n * sizeof(double2)) return false;
         }
     }
     return true;

@@ -89,7 +89,10 @@ struct PassPlan
     DevArray<int4>                   par_group;
     DevArray<int2>                   par_ent;
     int                              npar_src = 0, npar_tgt = 0;
-    int                              spec_slots = 0;  // block spectra are of slots below this
+    int                              spec_slots = 0;  // block spectra are of slots below this,
+    int                              top_slots = 0;   // those below the base level of slots below this
+    int                              nfwd_top = 0;    // the first of fwd, below the base level
+    int                              ninv_base = 0;   // inv starts with these, at the base level or above
     long                             par_nfwd = 0, par_ninv = 0, par_npairs = 0;
     MacLevelPlan                     par_stats;
     long                             npairs = 0;
@@ -358,10 +361,11 @@ class GpuSolver
     PassPlan& pass(int L, int nl, bool neighbor_only);
     PassPlan& pass_idx(int L, int idx, bool neighbor_only);
     static int pass_key(int L, int idx, bool neighbor_only) { return (L * 64 + idx) * 2 + (neighbor_only ? 1 : 0); }
-    bool      has_ghat(bool laplace, int d, double alpha) const;
+    bool      has_ghat(bool laplace, int d, double alpha, int prec) const;
+    int       mac_precision(const MacLevelPlan& m) const;  // of the spectra of the level's blocks
     void      build_separable(PassPlan& p, std::vector<char>& done);
     void      prepare_pass(PassPlan& p);  // kernel spectra of one Laplace pass
-    void      reserve_parents(const PassPlan& p, int k);
+    void      reserve_extra(const PassPlan& p, int k);
     const double2* parent_ghat();
     const double* if_iv(double alpha);
     const DevArray<int>& face_clean_list(int kind, int level, bool leaf_only);
@@ -376,7 +380,7 @@ class GpuSolver
     Batch     batch(int k) const;
     double2*    ghat_laplace(int d);
     double2*    ghat_if(double alpha);
-    const void* ghat(bool laplace, int d, double alpha);  // in the current precision
+    const void* ghat(bool laplace, int d, double alpha, int prec);  // in the current precision
     void       fill_zero(double* f, const Batch& b = {});
     int        forward_legs() const;  // arithmetic of the forward / inverse transforms' legs
     int        inverse_legs() const;
@@ -445,21 +449,22 @@ class GpuSolver
     };
     WorkPtrs wp_;
     // The spectra of one pass within that memory: source and target spectra of
-    // blocks, component c at c * b.sstride, and the rest.
+    // blocks (component c at c * b.sstride), with FP32 spectra those below the
+    // base level apart (FP64, at c * btop.sstride), and the rest.
     struct SpecPtrs
     {
-        void * sspec, *tspec, *rest;
-        size_t rest_bytes;
-        Batch  b;
+        void * sspec, *tspec, *stop, *ttop, *rest;
+        size_t rest_bytes, extra_bytes = 0;
+        Batch  b, btop;
     };
+    SpecPtrs spectra(const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes, void* extra) const;
+    SpecPtrs region_spectra(const PassPlan& p, int prec) const;
+    SpecPtrs pass_spectra(const PassPlan& p, const Batch& b);
     void     run_parents(PassPlan& p, double scale, const SpecPtrs& sp);
-    SpecPtrs spectra(const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes) const;
-    bool     fits_region(const PassPlan& p) const;
     bool     amr2amr(const PassPlan& p) const;
     size_t   spec_region_bytes(int prec) const;
-    // Scratch of whole parents that do not fit the rest: of the largest such
-    // pass run, and (never moved while the tree is loaded) of the allocation-free
-    // solve's.
+    // Spectra that do not fit: of the largest such pass run, and (never moved
+    // while the tree is loaded) of the allocation-free solve's.
     DevArray<double2> par_extra_, par_one_;
     DevArray<double2> par_ghat_;
     bool                                          graphs_ = false;

@@ -379,7 +379,7 @@ void GpuSolver::step_prepare(const double alpha[3], int refresh)
         // the STREAM pass: it can have more parents than any pass of the solves
         PassPlan& sp = pass_idx(base_level_, fmm_mask_idx_gen(MASK_STREAM), false);
         prepare_pass(sp);
-        reserve_parents(sp, 1);
+        reserve_extra(sp, 1);
         if (refresh == 1) prepare_if(0.0);
         sync();
     }

@@ -459,15 +459,17 @@ struct LegSplit
 // is the other way round).  Twiddles come from a table T[k][j] = w^(j k), so the inner loops
 // carry no modular index arithmetic.  Arithmetic and LDS intermediates are
 // FP64; the spectrum is stored as T (double: plain FP64 path; float: mixed
-// path).
+// path, where the first `top.count` blocks go to the FP64 spectra `top`: a
+// launch of their own takes 45 us for however few).
 constexpr int kFwdThreads = 1024;
 
 template<int N, class T>
 __global__ __launch_bounds__(kFwdThreads) void k_forward_dft(const double* __restrict__ field,
     const double* __restrict__ field_in, int split, const int* __restrict__ slots, int count, int ncomp,
-    typename Cx<T>::type* __restrict__ spec, long fcs, long scs)
+    typename Cx<T>::type* __restrict__ spec, long fcs, long scs, TopSpectra top)
 {
     using G = Geo<N>;
+    using C = typename Cx<T>::type;
     constexpr int P = G::P, H = G::H, GS = DftPlan<N>::GS;
     static_assert(GS >= 1 && H % GS == 0, "groups of whole kx-planes");
     using SX = LegSplit<N * N, GS, kFwdThreads>;   // x leg: lines (z, y), outputs kx in the group
@@ -491,7 +493,9 @@ __global__ __launch_bounds__(kFwdThreads) void k_forward_dft(const double* __res
         const int     c = item / count, b = item - c * count, slot = slots[b];
         const bool    ring0 = b >= split;  // read field_in, its boundary ring taken as zero
         const double* in = (ring0 ? field_in : field) + c * fcs + (size_t)slot * G::N3;
-        typename Cx<T>::type* out = spec + c * scs + (size_t)slot * G::NF;
+        const bool    fine = sizeof(T) == 4 && b < top.count;  // the same for the whole workgroup
+        char*         out = fine ? reinterpret_cast<char*>(top.spec + c * top.stride + (size_t)slot * G::NF)
+                                 : reinterpret_cast<char*>(spec + c * scs + (size_t)slot * G::NF);
         for (int kx0 = 0; kx0 < H; kx0 += GS)
         {
             // x leg: real line (z, y) of N points -> planes g in [g0, g0 + per)
@@ -564,10 +568,19 @@ __global__ __launch_bounds__(kFwdThreads) void k_forward_dft(const double* __res
                     for (int o = 0; o < SZ::per; ++o)
                         if (k0 + o < P) cmac_conj(a, Tw[(k0 + o) * N + z], sr[o], si[o]);
                 }
-                typename Cx<T>::type* o = out + (size_t)(kx * P + ky) * P + k0;
+                char* to = out + ((kx * P + ky) * P + k0) * (fine ? (int)sizeof(double2) : (int)sizeof(C));
+                if (fine)
+                {
 #pragma unroll
-                for (int q = 0; q < SZ::per; ++q)
-                    if (k0 + q < P) o[q] = Cx<T>::make((T)sr[q], (T)si[q]);
+                    for (int q = 0; q < SZ::per; ++q)
+                        if (k0 + q < P) reinterpret_cast<double2*>(to)[q] = make_double2(sr[q], si[q]);
+                }
+                else
+                {
+#pragma unroll
+                    for (int q = 0; q < SZ::per; ++q)
+                        if (k0 + q < P) reinterpret_cast<C*>(to)[q] = Cx<T>::make((T)sr[q], (T)si[q]);
+                }
             }
             __syncthreads();
         }
@@ -581,14 +594,14 @@ __global__ __launch_bounds__(kFwdThreads) void k_forward_dft(const double* __res
 // is split over the workgroup's kInvThreads threads as LegSplit (twice the
 // forward kernel's threads: the same LDS footprint then holds 12 waves per
 // CU).  Twiddles come from a table I[o][k] = w^((n-1+o) k).  FP64 arithmetic;
-// the spectrum is read as T (double: plain FP64 path; float: mixed path) and
-// widened on load.
+// the spectrum is read as T (double: plain FP64 path; float: mixed path, where
+// the last `top.count` blocks' are the FP64 spectra `top`) and widened on load.
 constexpr int kInvThreads = 768;
 
 template<int N, class T>
 __global__ __launch_bounds__(kInvThreads) void k_inverse_dft(const typename Cx<T>::type* __restrict__ spec,
     const int* __restrict__ slots, int count, double* __restrict__ field, double scale, int accumulate, long scs,
-    long fcs)
+    long fcs, TopSpectra top)
 {
     using G = Geo<N>;
     constexpr int P = G::P, H = G::H, GS = DftPlan<N>::GS;
@@ -622,27 +635,33 @@ __global__ __launch_bounds__(kInvThreads) void k_inverse_dft(const typename Cx<T
     for (int kx0 = 0; kx0 < H; kx0 += GS)
     {
         // z leg: row (g, ky) of P frequencies -> window points z in [z0, z0 + per)
-        for (int it = threadIdx.x; it < SZ::items; it += kInvThreads)
-        {
-            const int      part = it / SZ::lines, line = it - part * SZ::lines;
-            const int      g = line / P, ky = line - g * P, kx = kx0 + g;
-            const int      z0 = part * SZ::per;
-            const typename Cx<T>::type* row = in + (size_t)(kx * P + ky) * P;
-            double         sr[SZ::per], si[SZ::per];
-#pragma unroll
-            for (int o = 0; o < SZ::per; ++o) sr[o] = si[o] = 0.0;
-#pragma unroll 7
-            for (int kz = 0; kz < P; ++kz)
+        const auto z_leg = [&](const auto* from) {
+            for (int it = threadIdx.x; it < SZ::items; it += kInvThreads)
             {
-                const double2 a = widen(row[kz]);
+                const int   part = it / SZ::lines, line = it - part * SZ::lines;
+                const int   g = line / P, ky = line - g * P, kx = kx0 + g;
+                const int   z0 = part * SZ::per;
+                const auto* row = from + (size_t)(kx * P + ky) * P;
+                double      sr[SZ::per], si[SZ::per];
+#pragma unroll
+                for (int o = 0; o < SZ::per; ++o) sr[o] = si[o] = 0.0;
+#pragma unroll 7
+                for (int kz = 0; kz < P; ++kz)
+                {
+                    const double2 a = widen(row[kz]);
+#pragma unroll
+                    for (int o = 0; o < SZ::per; ++o)
+                        if (z0 + o < N) cmac(a, Iw[(z0 + o) * P + kz], sr[o], si[o]);
+                }
 #pragma unroll
                 for (int o = 0; o < SZ::per; ++o)
-                    if (z0 + o < N) cmac(a, Iw[(z0 + o) * P + kz], sr[o], si[o]);
+                    if (z0 + o < N) U[(g * P + ky) * N + z0 + o] = make_double2(sr[o], si[o]);
             }
-#pragma unroll
-            for (int o = 0; o < SZ::per; ++o)
-                if (z0 + o < N) U[(g * P + ky) * N + z0 + o] = make_double2(sr[o], si[o]);
-        }
+        };
+        if (sizeof(T) == 4 && b >= count - top.count)  // the same for the whole workgroup
+            z_leg(static_cast<const double2*>(top.spec) + blockIdx.y * top.stride + (size_t)slot * G::NF);
+        else
+            z_leg(in);
         __syncthreads();
         // y leg: line (g, z) of P frequencies -> window points y in [y0, y0 + per)
         for (int it = threadIdx.x; it < SY::items; it += kInvThreads)
@@ -1350,32 +1369,32 @@ inline int resident_grid(F kernel, int threads, long items)
 template<int N> struct RunFwd
 {
     static void run(hipStream_t s, int prec, const double* f, const double* fin, int split, const int* slots,
-        int count, void* spec, const Batch& b)
+        int count, void* spec, const Batch& b, const TopSpectra& top)
     {
         const long items = static_cast<long>(count) * b.k;
         if (prec == 0)
             hipLaunchKernelGGL((k_forward_dft<N, double>),
                 dim3(b.dft_grid ? items : resident_grid(k_forward_dft<N, double>, kFwdThreads, items)),
-                dim3(kFwdThreads), 0, s, f, fin, split, slots, count, b.k, (double2*)spec, b.fstride, b.sstride);
+                dim3(kFwdThreads), 0, s, f, fin, split, slots, count, b.k, (double2*)spec, b.fstride, b.sstride, top);
         else
             hipLaunchKernelGGL((k_forward_dft<N, float>),
                 dim3(b.dft_grid ? items : resident_grid(k_forward_dft<N, float>, kFwdThreads, items)),
-                dim3(kFwdThreads), 0, s, f, fin, split, slots, count, b.k, (float2*)spec, b.fstride, b.sstride);
+                dim3(kFwdThreads), 0, s, f, fin, split, slots, count, b.k, (float2*)spec, b.fstride, b.sstride, top);
     }
 };
 template<int N> struct RunInv
 {
     static void run(hipStream_t s, int prec, const void* spec, const int* slots, int count, double* f, double scale,
-        int accumulate, const Batch& b)
+        int accumulate, const Batch& b, const TopSpectra& top)
     {
         // One workgroup per (block, component): a workgroup looping over
         // blocks, as the forward transform does, measured slower here.
         if (prec == 0)
             hipLaunchKernelGGL((k_inverse_dft<N, double>), dim3(count, b.k), dim3(kInvThreads), 0, s,
-                (const double2*)spec, slots, count, f, scale, accumulate, b.sstride, b.fstride);
+                (const double2*)spec, slots, count, f, scale, accumulate, b.sstride, b.fstride, top);
         else
             hipLaunchKernelGGL((k_inverse_dft<N, float>), dim3(count, b.k), dim3(kInvThreads), 0, s,
-                (const float2*)spec, slots, count, f, scale, accumulate, b.sstride, b.fstride);
+                (const float2*)spec, slots, count, f, scale, accumulate, b.sstride, b.fstride, top);
     }
 };
 // Workgroup size of a MAC launch: every (group, component) pair of the launch
@@ -1503,28 +1522,46 @@ void correction_stencil(hipStream_t s, int n, const double* t, double* c, const 
 {
     if (count > 0) dispatch_n<RunStencil>(n, s, t, c, slots, count, inv_dx2, omega2, b);
 }
+// A launch of the top blocks alone, in plain FP64: where the precision's own
+// transforms cannot hold them.
+static Batch top_batch(const Batch& b, const TopSpectra& top)
+{
+    Batch t = b;
+    t.sstride = top.stride;
+    return t;
+}
 void forward_dft(hipStream_t s, int n, int prec, const double* field, const int* slots, int count, void* spec,
-    const Batch& b, const double* field_in, int split)
+    const Batch& b, const double* field_in, int split, const TopSpectra& top)
 {
     if (split < 0) split = count;
     if (split > count) throw std::invalid_argument("forward_dft: split outside the block list");
     if (split < count && !field_in) throw std::invalid_argument("forward_dft: no field for the interior-read blocks");
+    if (top.count > split || (prec == kPrecFp64 && top.count)) throw std::invalid_argument("forward_dft: top blocks");
     if (prec_mfma(prec))
     {
-        forward_dft_mfma(s, n, prec, field, slots, count, static_cast<float2*>(spec), b, field_in, split);
+        if (top.count)
+            dispatch_n<RunFwd>(
+                n, s, kPrecFp64, field, field_in, top.count, slots, top.count, top.spec, top_batch(b, top), TopSpectra{});
+        forward_dft_mfma(s, n, prec, field, slots + top.count, count - top.count, static_cast<float2*>(spec), b, field_in,
+            split - top.count);
         return;
     }
-    if (count > 0) dispatch_n<RunFwd>(n, s, prec, field, field_in, split, slots, count, spec, b);
+    if (count > 0) dispatch_n<RunFwd>(n, s, prec, field, field_in, split, slots, count, spec, b, top);
 }
 void inverse_dft(hipStream_t s, int n, int prec, const void* spec, const int* slots, int count, double* field,
-    double scale, bool accumulate, const Batch& b)
+    double scale, bool accumulate, const Batch& b, const TopSpectra& top)
 {
+    if (top.count > count || (prec == kPrecFp64 && top.count)) throw std::invalid_argument("inverse_dft: top blocks");
     if (prec_mfma(prec))
     {
-        inverse_dft_mfma(s, n, prec, static_cast<const float2*>(spec), slots, count, field, scale, accumulate, b);
+        inverse_dft_mfma(
+            s, n, prec, static_cast<const float2*>(spec), slots, count - top.count, field, scale, accumulate, b);
+        if (top.count)
+            dispatch_n<RunInv>(n, s, kPrecFp64, static_cast<const void*>(top.spec), slots + count - top.count, top.count,
+                field, scale, accumulate ? 1 : 0, top_batch(b, top), TopSpectra{});
         return;
     }
-    if (count > 0) dispatch_n<RunInv>(n, s, prec, spec, slots, count, field, scale, accumulate ? 1 : 0, b);
+    if (count > 0) dispatch_n<RunInv>(n, s, prec, spec, slots, count, field, scale, accumulate ? 1 : 0, b, top);
 }
 void spectral_mac(hipStream_t s, int n, int prec, const MacGroup* groups, int ngroups, const MacSrc* srcs,
     const uint4* rowoff, const int* olist, int nused, bool compact, const void* ghat, const void* sspec,

@@ -179,6 +179,15 @@ __device__ __attribute__((always_inline)) inline void each_point(Load load, Stor
     }
 }
 
+// FP64 spectra of some of a transform's blocks beside FP32 ones of the others
+// (component c at c * stride).
+struct TopSpectra
+{
+    double2* spec = nullptr;
+    long     stride = 0;
+    int      count = 0;
+};
+
 namespace launch {
 
 bool supported_n(int n);
@@ -217,12 +226,13 @@ void correction_stencil(hipStream_t s, int n, const double* target_tmp, double* 
 // prec 2-5 (prec_mfma): spectra and MAC as prec 1, the DFT legs on the
 // matrix cores (forward_dft_mfma / inverse_dft_mfma).
 // Blocks slots[split..count) are read from field_in with their boundary ring
-// taken as zero, the others from field.
+// taken as zero, the others from field.  top (prec > 0): the spectra of the
+// first top.count blocks, of the last top.count in inverse_dft; their legs are FP64.
 void forward_dft(hipStream_t s, int n, int prec, const double* field, const int* slots, int count, void* spec,
-    const Batch& b = {}, const double* field_in = nullptr, int split = -1);
+    const Batch& b = {}, const double* field_in = nullptr, int split = -1, const TopSpectra& top = {});
 // Writes (accumulate: adds into) every point of each listed field block.
 void inverse_dft(hipStream_t s, int n, int prec, const void* spec, const int* slots, int count, double* field,
-    double scale, bool accumulate, const Batch& b = {});
+    double scale, bool accumulate, const Batch& b = {}, const TopSpectra& top = {});
 // olist[nused]: the offsets (0..342, o = (ox+3) + 7 (oy+3) + 49 (oz+3)) the
 // launch's entries use.  A compact launch (nused <= kMacCompactMax) stages
 // only those rows, row i = olist[i]; otherwise row o = offset o.  Row nrows

@@ -298,10 +298,25 @@ __device__ inline size_t spec_at(int f, int chunk0, int row, int rows)
 // in.  Frequencies are independent of each other between the z legs, so a
 // pass whose spectra do not fit its scratch takes them some planes at a time;
 // an outer chunk's other planes are neither written nor read.
+//
+// The storage type of a plane (T double: FP64 for all): with T float, planes
+// below zl are FP64 and the others FP32, the FP32 chunks behind the FP64
+// ones; a chunk that holds planes of both is stored as both.
 struct Slice
 {
-    int z0, nz, chunk0, nchunk;
+    int z0, nz, zl;
+    int chunk0, nchunk;    // of the planes [z0, zl)
+    int chunk0f, nchunkf;  // of the planes [zl, z0 + nz)
 };
+// The FP32 chunks of a spectrum array.
+__device__ inline const float2* low_part(const double2* spec, const Slice& sl, int rows)
+{
+    return reinterpret_cast<const float2*>(spec + (size_t)sl.nchunk * rows * 64);
+}
+__device__ inline float2* low_part(double2* spec, const Slice& sl, int rows)
+{
+    return reinterpret_cast<float2*>(spec + (size_t)sl.nchunk * rows * 64);
+}
 
 // ---------------------------------------------------------------------------
 // Forward z leg (real to half spectrum): mid[item][kz][y][x], item = component
@@ -413,7 +428,7 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_fwd_z(const double* __r
 // ---------------------------------------------------------------------------
 template<int N, class T>
 __global__ __launch_bounds__(Par<N>::T) __attribute__((amdgpu_waves_per_eu(5))) void k_parent_fwd_plane(
-    const double2* __restrict__ mid, typename Spec<T>::C* __restrict__ spec, int rows, Slice sl)
+    const double2* __restrict__ mid, double2* __restrict__ spec, int rows, Slice sl)
 {
     using G = Par<N>;
     constexpr int      M = G::M, P = G::P, R1 = G::R1, R2 = G::R2, PS = G::PS;
@@ -439,9 +454,17 @@ __global__ __launch_bounds__(Par<N>::T) __attribute__((amdgpu_waves_per_eu(5))) 
         const int k1 = l / P, qy = l - k1 * P;
         leg_roots<R1, -1>(k1, tab, w);
         forward_first<N>(w, v, [&](int n) { return Y[n * PS + qy]; });
-        small_dft<R2, -1>(v, [&](int k2, double2 X) {
-            spec[spec_at(kz * G::PP + (k2 * R1 + k1) * P + qy, sl.chunk0, row, rows)] = Spec<T>::put(X);
-        });
+        const int f = kz * G::PP + k1 * P + qy;
+        if (sizeof(T) == 8 || kz < sl.zl)  // the same for the whole workgroup
+            small_dft<R2, -1>(
+                v, [&](int k2, double2 X) { spec[spec_at(f + k2 * (R1 * P), sl.chunk0, row, rows)] = X; });
+        else
+        {
+            float2* out = low_part(spec, sl, rows);
+            small_dft<R2, -1>(v, [&](int k2, double2 X) {
+                out[spec_at(f + k2 * (R1 * P), sl.chunk0f, row, rows)] = Spec<float>::put(X);
+            });
+        }
     }
 }
 
@@ -483,24 +506,13 @@ __device__ inline void mac_entries(const int2* __restrict__ ent, int& e, int end
     }
 }
 
+// The products of one chunk: T is its storage type.
 template<class T>
-__global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int4* __restrict__ group,
-    const int* __restrict__ begin, const int2* __restrict__ ent, int ngroup, int ntgt, int nsrc, int ncomp, const double2* __restrict__ ghat,
-    const typename Spec<T>::C* __restrict__ sspec, typename Spec<T>::C* __restrict__ tspec, Slice sl, int nseg)
+__device__ inline void mac_chunk(const int4* __restrict__ group, const int* __restrict__ begin,
+    const int2* __restrict__ ent, int ngroup, int ntgt, int nsrc, int ncomp, const double2* Gs,
+    const typename Spec<T>::C* __restrict__ sspec, typename Spec<T>::C* __restrict__ tspec, int chunk, int seg, int nseg)
 {
-    __shared__ double2 Gs[(kParentNone + 1) * 64];
-    const int          r = blockIdx.x >> 3, chunk = (r / nseg) * 8 + (blockIdx.x & 7), seg = r % nseg;
-    if (chunk >= sl.nchunk) return;  // the whole workgroup
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (wave == kMacWaves - 1) Gs[kParentNone * 64 + lane] = make_double2(0.0, 0.0);
-    for (int o = wave; o < 27; o += kMacWaves)
-    {
-        // stored: offsets 13 (own parent) to 26; offset o < 13 is the opposite of 26 - o
-        double2 g = ghat[((size_t)(sl.chunk0 + chunk) * 14 + (o < 13 ? 13 - o : o - 13)) * 64 + lane];
-        if (o < 13) g.y = -g.y;
-        Gs[o * 64 + lane] = g;
-    }
-    __syncthreads();
     const int npair = ngroup * ncomp, per = (npair + nseg - 1) / nseg, lo = seg * per, hi = min(lo + per, npair);
     for (int pr = lo + wave; pr < hi; pr += kMacWaves)
     {
@@ -521,6 +533,32 @@ __global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int4* __res
         if (to.z >= 0) tp[(size_t)to.z * 64] = Spec<T>::put(acc[2]);
         if (to.w >= 0) tp[(size_t)to.w * 64] = Spec<T>::put(acc[3]);
     }
+}
+
+template<class T>
+__global__ __launch_bounds__(64 * kMacWaves) void k_parent_mac(const int4* __restrict__ group,
+    const int* __restrict__ begin, const int2* __restrict__ ent, int ngroup, int ntgt, int nsrc, int ncomp, const double2* __restrict__ ghat,
+    const double2* __restrict__ sspec, double2* __restrict__ tspec, Slice sl, int nseg)
+{
+    __shared__ double2 Gs[(kParentNone + 1) * 64];
+    const int          r = blockIdx.x >> 3, chunk = (r / nseg) * 8 + (blockIdx.x & 7), seg = r % nseg;
+    if (chunk >= sl.nchunk + sl.nchunkf) return;  // the whole workgroup
+    const bool fine = sizeof(T) == 8 || chunk < sl.nchunk;
+    const int  lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int  gc = fine ? sl.chunk0 + chunk : sl.chunk0f + chunk - sl.nchunk;  // chunk of the whole spectrum
+    if (wave == kMacWaves - 1) Gs[kParentNone * 64 + lane] = make_double2(0.0, 0.0);
+    for (int o = wave; o < 27; o += kMacWaves)
+    {
+        // stored: offsets 13 (own parent) to 26; offset o < 13 is the opposite of 26 - o
+        double2 g = ghat[((size_t)gc * 14 + (o < 13 ? 13 - o : o - 13)) * 64 + lane];
+        if (o < 13) g.y = -g.y;
+        Gs[o * 64 + lane] = g;
+    }
+    __syncthreads();
+    if (fine) mac_chunk<double>(group, begin, ent, ngroup, ntgt, nsrc, ncomp, Gs, sspec, tspec, chunk, seg, nseg);
+    else
+        mac_chunk<float>(group, begin, ent, ngroup, ntgt, nsrc, ncomp, Gs, low_part(sspec, sl, nsrc * ncomp),
+            low_part(tspec, sl, ntgt * ncomp), chunk - sl.nchunk, seg, nseg);
 }
 
 // ---------------------------------------------------------------------------
@@ -544,7 +582,7 @@ __device__ inline int window(int a, int b)  // window point of (a, b), W or more
 
 template<int N, class T>
 __global__ __launch_bounds__(Par<N>::T) void k_parent_inv_plane(
-    const typename Spec<T>::C* __restrict__ spec, double2* __restrict__ mid, int rows, Slice sl)
+    const double2* __restrict__ spec, double2* __restrict__ mid, int rows, Slice sl)
 {
     using G = Par<N>;
     constexpr int      P = G::P, R1 = G::R1, R2 = G::R2, W = G::W, WS = G::WS;
@@ -553,14 +591,23 @@ __global__ __launch_bounds__(Par<N>::T) void k_parent_inv_plane(
     const int          l = threadIdx.x, zl = blockIdx.x / rows, row = blockIdx.x - zl * rows, kz = sl.z0 + zl;
     mid += ((size_t)row * G::H + kz) * (W * W);
     double2 u[R1], v[R2];
-    for (int it = l; it < R2 * P; it += G::T)
+    const auto first = [&](auto load) {
+        for (int it = l; it < R2 * P; it += G::T)
+        {
+            const int k2 = it / P, at = k2 * (R1 * P) + it - k2 * P;
+#pragma unroll
+            for (int k = 0; k < R1; ++k) u[k] = load(kz * G::PP + at + k * P);
+            inverse_first<R1>(u);
+#pragma unroll
+            for (int k = 0; k < R1; ++k) buf[at + k * P] = u[k];
+        }
+    };
+    if (sizeof(T) == 8 || kz < sl.zl)  // the same for the whole workgroup
+        first([&](int f) { return spec[spec_at(f, sl.chunk0, row, rows)]; });
+    else
     {
-        const int k2 = it / P, at = k2 * (R1 * P) + it - k2 * P;
-#pragma unroll
-        for (int k = 0; k < R1; ++k) u[k] = Spec<T>::get(spec[spec_at(kz * G::PP + at + k * P, sl.chunk0, row, rows)]);
-        inverse_first<R1>(u);
-#pragma unroll
-        for (int k = 0; k < R1; ++k) buf[at + k * P] = u[k];
+        const float2* in = low_part(spec, sl, rows);
+        first([&](int f) { return Spec<float>::get(in[spec_at(f, sl.chunk0f, row, rows)]); });
     }
     __syncthreads();
     const int a = l / P, qy = l - a * P;
@@ -742,11 +789,22 @@ __global__ __launch_bounds__(kLineThreads) void k_parent_ghat_leg(
 // Launches
 // ---------------------------------------------------------------------------
 inline unsigned blocks_of(long total, int per) { return (unsigned)((total + per - 1) / per); }
+
+// With FP32 spectra the first kz planes are FP64 all the same.  The low
+// frequencies are the ones that count: the kernel falls off with the square
+// of the frequency, and the rounding of one value near zero frequency reaches the
+// whole parent in phase.  18 trees of 73 to 4290 blocks and three components each,
+// error against FP64 as a multiple of that of block transforms (mean, largest; the
+// coarser levels' part taken out as far as spectra() does): no plane 0.41,
+// 1.4; two 0.14, 0.9; three 0.11, 1.3.  4290 blocks, three components: 9.69, 9.74
+// and 9.79 ms.
+constexpr int kFinePlanes = 2;
+
 constexpr size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 // Where a pass keeps its spectra and columns, for ns source and nt target
-// parents (times components) and values of `elem` bytes, in bytes from the
-// start of its scratch.  All planes in one round: the columns of the forward
+// parents (times components), in bytes from the start of its scratch; planes
+// from `fine` on are FP32.  All planes in one round: the columns of the forward
 // legs lie where the target spectra come later, those of the inverse legs
 // where the source spectra were.  In rounds of nz planes: the inverse legs'
 // columns apart, since the last leg needs all planes; the forward z leg runs
@@ -757,28 +815,33 @@ struct Layout
     int    nz = 0;  // planes a round; 0: does not fit
     size_t mid_s = 0, mid_t = 0, sspec = 0, tspec = 0, bytes = 0;
 
-    static Slice slice(int z0, int nz)
+    static Slice slice(int z0, int nz, int fine)
     {
-        nz = std::min(nz, G::H - z0);
-        const int c0 = z0 * G::PP / 64;
-        return Slice{z0, nz, c0, ((z0 + nz) * G::PP + 63) / 64 - c0};
+        const int z1 = std::min(z0 + nz, G::H), zl = std::min(std::max(z0, fine), z1);
+        auto      first = [](int z) { return z * G::PP / 64; };
+        auto      count = [&](int a, int b) { return a < b ? (b * G::PP + 63) / 64 - first(a) : 0; };
+        return Slice{z0, z1 - z0, zl, first(z0), count(z0, zl), first(zl), count(zl, z1)};
     }
-    Layout(long ns, long nt, size_t elem, int planes) : nz(planes)
+    Layout(long ns, long nt, int fine, int planes) : nz(planes)
     {
-        size_t chunks = 0;
-        for (int z0 = 0; z0 < G::H; z0 += nz) chunks = std::max<size_t>(chunks, slice(z0, nz).nchunk);
-        const size_t S = round256(ns * chunks * 64 * elem), T = round256(nt * chunks * 64 * elem);
+        size_t line = 0;  // bytes of a parent
+        for (int z0 = 0; z0 < G::H; z0 += nz)
+        {
+            const Slice sl = slice(z0, nz, fine);
+            line = std::max(line, 64 * (sl.nchunk * sizeof(double2) + sl.nchunkf * sizeof(float2)));
+        }
+        const size_t S = round256(ns * line), T = round256(nt * line);
         const size_t ms = round256((size_t)ns * nz * G::M * G::M * sizeof(double2));
         const size_t mt = round256((size_t)nt * G::H * G::W * G::W * sizeof(double2));
         sspec = nz == G::H ? 0 : mt;
         tspec = mid_s = nz == G::H ? std::max(S, mt) : mt + S;
         bytes = tspec + std::max(T, ms);
     }
-    static Layout fit(long ns, long nt, size_t elem, size_t room)
+    static Layout fit(long ns, long nt, int fine, size_t room)
     {
-        Layout l(ns, nt, elem, G::H);
+        Layout l(ns, nt, fine, G::H);
         for (int z = 2; l.bytes > room && z <= G::H; ++z)  // z rounds
-            if ((G::H + z - 1) / z < l.nz) l = Layout(ns, nt, elem, (G::H + z - 1) / z);
+            if ((G::H + z - 1) / z < l.nz) l = Layout(ns, nt, fine, (G::H + z - 1) / z);
         if (l.bytes > room) l.nz = 0;
         return l;
     }
@@ -792,13 +855,13 @@ struct Run
     template<class T>
     static void pass(hipStream_t s, const ParentPass& p, const double* src, double* dst, double scale, const Batch& b)
     {
-        using C = typename Spec<T>::C;
         const long ns = (long)p.nsrc * b.k, nt = (long)p.ntgt * b.k;
-        const L    l = L::fit(ns, nt, sizeof(C), p.bytes);
+        const int  fine = fine_planes(sizeof(T) == 4);
+        const L    l = L::fit(ns, nt, fine, p.bytes);
         if (l.nz == 0) throw std::logic_error("parent_pass: scratch too small");
         char*    at = static_cast<char*>(p.scratch);
-        double2 *mid_s = reinterpret_cast<double2*>(at + l.mid_s), *mid_t = reinterpret_cast<double2*>(at + l.mid_t);
-        C *      sspec = reinterpret_cast<C*>(at + l.sspec), *tspec = reinterpret_cast<C*>(at + l.tspec);
+        auto     to = [&](size_t o) { return reinterpret_cast<double2*>(at + o); };
+        double2 *mid_s = to(l.mid_s), *mid_t = to(l.mid_t), *sspec = to(l.sspec), *tspec = to(l.tspec);
         // (group, component) pairs a wave: fewer read the kernel values more often, more leave a chunk's
         // sources to L2 for longer (4290 blocks, 2 and 4 pairs: FP64 1.058 and 1.065 ms, with fewer blocks
         // 0.389 and 0.404; FP32, three components, 1.95 and 1.83)
@@ -807,7 +870,7 @@ struct Run
         const dim3 zgrid(blocks_of(ns * G::M * G::M, kLineThreads)), zthreads(kLineThreads);
         for (int z0 = 0; z0 < G::H; z0 += l.nz)
         {
-            const Slice sl = L::slice(z0, l.nz);
+            const Slice sl = L::slice(z0, l.nz, fine);
             if (l.nz == G::H)
                 hipLaunchKernelGGL((k_parent_fwd_z<N, false>), zgrid, zthreads, 0, s, src, b.fstride, p.src_child, p.nsrc,
                     b.k, mid_s, 0, G::H);
@@ -816,7 +879,7 @@ struct Run
                     b.k, mid_s, sl.z0, sl.nz);
             hipLaunchKernelGGL((k_parent_fwd_plane<N, T>), dim3((unsigned)(ns * sl.nz)), dim3(G::T), 0, s, mid_s, sspec,
                 (int)ns, sl);
-            hipLaunchKernelGGL(k_parent_mac<T>, dim3((unsigned)((sl.nchunk + 7) / 8 * 8 * nseg)), dim3(64 * kMacWaves), 0,
+            hipLaunchKernelGGL(k_parent_mac<T>, dim3((unsigned)((sl.nchunk + sl.nchunkf + 7) / 8 * 8 * nseg)), dim3(64 * kMacWaves), 0,
                 s, p.group, p.begin, p.entries, p.ngroup, p.ntgt, p.nsrc, b.k, p.ghat, sspec, tspec, sl, nseg);
             hipLaunchKernelGGL(
                 (k_parent_inv_plane<N, T>), dim3((unsigned)(nt * sl.nz)), dim3(G::T), 0, s, tspec, mid_t, (int)nt, sl);
@@ -825,9 +888,11 @@ struct Run
             mid_t, p.tgt_child, p.ntgt, b.k, dst, b.fstride,
             scale / ((double)G::P * G::P * G::P));
     }
-    static size_t bytes(long ns, long nt, size_t elem, size_t room)
+    static constexpr int fine_planes(bool fp32) { return fp32 ? kFinePlanes : G::H; }
+    static size_t bytes(long ns, long nt, bool fp32, size_t room)
     {
-        const L l = room ? L::fit(ns, nt, elem, room) : L(ns, nt, elem, G::H);
+        const int fine = fine_planes(fp32);
+        const L   l = room ? L::fit(ns, nt, fine, room) : L(ns, nt, fine, G::H);
         return l.nz ? l.bytes : 0;
     }
     static void spectra(hipStream_t s, const double* sample, double2* a, double2* b, double2* ghat)
@@ -878,8 +943,7 @@ void parent_pass(hipStream_t s, int n, int prec, const ParentPass& p, const doub
 }
 size_t parent_bytes(int n, int prec, long nsrc, long ntgt, size_t room)
 {
-    const size_t elem = prec == 0 ? sizeof(double2) : sizeof(float2);
-    return on_n(n, [&](auto r) { return decltype(r)::bytes(nsrc, ntgt, elem, room); });
+    return on_n(n, [&](auto r) { return decltype(r)::bytes(nsrc, ntgt, prec != 0, room); });
 }
 void parent_spectra(hipStream_t s, int n, const double* sample, double2* a, double2* b, double2* ghat)
 {

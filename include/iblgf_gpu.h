@@ -365,9 +365,12 @@ enum iblgf_precision
     IBLGF_PREC_MIXED = 1,  /* source, kernel and target spectra stored FP32 (kernel spectra
                               generated in FP64; target spectra accumulated in FP64 and rounded
                               once on store), MAC products in FP32; DFT arithmetic, fields and
-                              cross-level transfers FP64 */
-    /* Spectra, MAC, fields and transfers as IBLGF_PREC_MIXED, every 1-D DFT
-     * leg a GEMM on the matrix cores with FP32 intermediates: */
+                              cross-level transfers FP64.  FP64 throughout, in this and the
+                              following precisions: the blocks below the base level, and of
+                              whole parents (the finest level) the kernel spectra, the products
+                              and the first planes of the spectra */
+    /* Spectra, MAC, fields and transfers as IBLGF_PREC_MIXED, every other 1-D
+     * leg of block transforms a GEMM on the matrix cores with FP32 intermediates: */
     IBLGF_PREC_BF16X3 = 2,  /* BF16 hi/lo split, three products, FP32 accumulation */
     IBLGF_PREC_FP16X3 = 3,  /* FP16 hi/lo split of power-of-two scaled lines, three products,
                                FP32 accumulation */

@@ -8,7 +8,8 @@ import numpy as np
 import pytest
 import torch
 
-from iblgf_amd import FLAG_LEAF, PREC_FP16X3_FORWARD, PREC_FP64, PREC_MIXED, PoissonSolver, Tree, lib, setups
+from iblgf_amd import (FLAG_LEAF, PREC_FP16X3_FORWARD, PREC_FP64, PREC_INT8X4, PREC_MIXED, PoissonSolver, Tree, lib,
+                       setups)
 
 pytestmark = pytest.mark.gpu
 
@@ -52,6 +53,17 @@ def test_groups_of_targets(oracle_mod, extent, precision, bound):
     that reach some of a group only."""
     print(f"case: whole-parent products in groups, {extent}^3 blocks, precision {precision}", flush=True)
     _check(oracle_mod, _uniform(extent, (7, 5, 3), box=16), 2, precision, bound)
+
+
+@pytest.mark.parametrize("precision", [PREC_MIXED, PREC_FP16X3_FORWARD, PREC_INT8X4])
+@pytest.mark.parametrize("extent", [6, 8, 10, 14, 16])
+def test_spectra_kept_in_fp64(oracle_mod, extent, precision):
+    """With FP32 spectra, FP64 ones below the base level (all coarser levels of
+    this mesh, in transforms of either kind) and for the first planes of whole
+    parents.  What is left is stored to 2^-24 of each value, once as a source and
+    once as a target: 1.2e-7."""
+    print(f"case: FP64 among FP32 spectra, {extent}^3 blocks, precision {precision}", flush=True)
+    _check(oracle_mod, _uniform(extent, (7, 5, 3), box=16), 2, precision, 1.2e-7)
 
 
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED, PREC_FP16X3_FORWARD])
