@@ -733,9 +733,16 @@ int iblgf_gpu_helm2d_table(const double* c, int nmodes, int nx, int ny, double* 
  * block pair of one level, include/iblgf/utilities/convolution.hpp:259-260
  * with the Helmholtz kernel):
  *   dst[k][t] = scale * sum_s table[k][|tj - sj|][|ti - si|] * src[k][s],
- * the sum over every cell s of the patch, directly or by transforms along x
- * (so dst satisfies (Lap_h - c^2) dst = scale * src at interior cells).  src and dst (nmodes x
- * ny x nx doubles) must differ; same limits as iblgf_gpu_helm2d_table. */
+ * the sum over every cell s of the patch, directly or (8 <= nx <= 512, ny >= 2,
+ * nx * ny >= 256) by transforms along x, so dst satisfies (Lap_h - c^2) dst =
+ * scale * src at interior cells.  The transforms' rounding is relative to whole
+ * rows, not to a cell's own terms: with P the power of two that they take
+ * (2 nx <= P < 4 nx, at least 64), a cell's error is within 3 log2(P) 2^-53
+ * times the sum over source rows of |row| |table row| (2-norms, of two
+ * neighbouring rows together).  Where screening has made the result smaller than
+ * that, it is noise; and a source value that is not finite spoils its whole
+ * mode.  src and dst (nmodes x ny x nx doubles) must differ; same limits as
+ * iblgf_gpu_helm2d_table. */
 int iblgf_gpu_helm2d_convolve(
     const double* table, int nmodes, int nx, int ny, const double* src, double* dst, double scale, void* stream);
 
