@@ -429,6 +429,15 @@ def helm2d_bench(steps, log, n=256, nmodes=8):
             "target_cells_per_s": cells * nmodes / (t_conv / 1e3)}
 
 
+def _digits(x):
+    """x with its floats rounded to seven significant digits."""
+    if isinstance(x, float):
+        return float(f"{x:.7g}")
+    if isinstance(x, dict):
+        return {k: _digits(v) for k, v in x.items()}
+    return [_digits(v) for v in x] if isinstance(x, (list, tuple)) else x
+
+
 def main():
     ap = argparse.ArgumentParser(description=__doc__)
     ap.add_argument("--gpus", type=int, default=1)
@@ -726,11 +735,14 @@ def main():
             "precision": {
                 None: "plain FP64 (no reduced-precision path met relative L2 1e-6)",
                 "mixed": ("mixed: source and kernel spectra stored FP32, multiplied in FP32 and accumulated in "
-                          "FP64 by the MAC, target spectra stored FP32; DFT arithmetic, fields and level sums FP64"),
+                          "FP64 by the MAC, target spectra stored FP32; DFT arithmetic, fields and level sums FP64; "
+                          "FP64 throughout below the base level, in the finest level's products and in the first "
+                          "planes of its spectra"),
                 "fp16x3forward": ("forward DFT legs as FP16 three-term GEMMs of power-of-two scaled lines on the "
                                   "matrix cores (FP32 accumulation, FP32 intermediates), inverse DFT legs FP64 on the "
                                   "vector ALUs; source, kernel and target spectra stored FP32, MAC products FP32 with "
-                                  "FP64 accumulation; fields and level sums FP64"),
+                                  "FP64 accumulation; fields and level sums FP64; FP64 throughout below the base level, "
+                                  "in the finest level's products and in the first planes of its spectra"),
                 "int8x4": ("DFT legs as INT8 digit-split GEMMs on the matrix cores (4 signed 7-bit digits, exact "
                            "INT32 sums), leg outputs FP32; spectra and MAC as the mixed path; fields and level sums "
                            "FP64"),
@@ -785,7 +797,19 @@ def main():
         # counts cover the FMM passes of one Laplace solve (each pass plan is built once)
         result["cpu_baseline"] = cpu_baseline(wl, srcs[0], counts, args.cpu_seconds)
     if rank == 0:
-        print(json.dumps(result))
+        # One line, short enough to be read from the end of a log: the other paths' class times and
+        # rooflines, autotuner reports and per-tree lists go to stderr, measured values to seven digits.
+        cfg = result["config"]
+        aside = [(cfg, k) for k in ("fp64_kernels", "fp64_batched_kernels", "fp64_roofline")]
+        for v in cfg["split_precision_batched"].values():
+            aside += [(v, "kernels"), (v, "dominant_roofline")]
+            v["relL2_vs_fp64_per_component"] = [e["relL2"] for e in v.pop("error_vs_fp64_per_component")]
+        aside += [(cfg.get("headline_autotune"), "report"), (cfg.get("learned_fcg"), "training")]
+        aside += [(cfg.get("forest_step"), k) for k in ("autotune_report", "blocks_per_tree", "target_blocks_per_tree")]
+        for holder, key in aside:
+            if holder and key in holder:
+                log(f"{key}: {json.dumps(_digits(holder.pop(key)))}")
+        print(json.dumps({k: v if k in ("value", "ms_per_step") else _digits(v) for k, v in result.items()}))
     return 0
 
 
