@@ -25,8 +25,6 @@ enum BlockOp
 
 namespace launch {
 
-// dst = op(src) over the interior of each listed block; fac = 1/dx (1/dx^2
-// for the Laplacian, (1/dx)*scale for the curl transpose).
 // Several levels in one launch: entry b takes the fac of the last level with begin <= b.
 struct LevelFac
 {
@@ -35,6 +33,8 @@ struct LevelFac
     int    begin[kMax];
     double fac[kMax];
 };
+// dst = op(src) over the interior of each listed block; fac = 1/dx (1/dx^2
+// for the Laplacian, (1/dx)*scale for the curl transpose).
 void block_op(hipStream_t s, int n, int op, const double* const src[3], double* const dst[3], const int* slots,
     int count, const LevelFac& fac);
 

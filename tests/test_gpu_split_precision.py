@@ -19,7 +19,7 @@ import numpy as np
 import pytest
 
 from iblgf_amd import (FLAG_LEAF, PREC_BF16X3, PREC_FP16, PREC_FP16X3, PREC_FP16X3_FORWARD, PREC_INT8X4,
-                       PoissonSolver, setups)
+                       PoissonSolver, Tree, lib, setups)
 
 pytestmark = pytest.mark.gpu
 
@@ -73,6 +73,30 @@ def test_split_precision_error_per_component(oracle_mod, extent, prec):
     # one component alone: bitwise the batched result
     solver.apply_lgf(fin[1], fout[0])
     assert np.array_equal(solver.download(fout[0]), got[1])
+
+
+@pytest.mark.parametrize("prec", [PREC_INT8X4, PREC_FP16X3, PREC_BF16X3, PREC_FP16, PREC_FP16X3_FORWARD])
+@pytest.mark.parametrize("extent", [6, 8, 10, 14, 16])
+def test_split_legs_of_every_block(oracle_mod, extent, prec):
+    """Whole parents and the levels below the base level leave the split legs
+    little to do on small trees.  On a level whose keys wrap every block goes
+    through them, in both directions (adding into its targets)."""
+    print(f"case: {NAME[prec]} legs of every block, keys that wrap, block extent {extent}", flush=True)
+    keys = [lib().iblgf_key_make(x, y, z, 1) for z in range(2) for y in range(2) for x in range(2)]
+    t = Tree.from_keys((0, 0, 0), extent, 1, 1.0, keys, [1] * 8).build_masks()
+    a, info = t.export(), t.info()
+    src = np.random.default_rng(extent).standard_normal((info["nblocks"],) + (t.n,) * 3)
+    solver = PoissonSolver(t)
+    solver.set_precision(prec)
+    fs, fd = solver.field(), solver.field()
+    solver.upload(fs, src)
+    solver.apply_lgf(fs, fd)
+    leaves = (a["flags"] & FLAG_LEAF) != 0
+    l2, mx = _rel(solver.download(fd)[leaves], oracle_mod.Tree(a, info, t.n).apply_lgf(src)[leaves])
+    print(f"{NAME[prec]} n={extent + 2}: relL2={l2:.3e} relmax={mx:.3e}", flush=True)
+    assert l2 < BOUND[prec]
+    # the legs did run: their rounding shows beside that of FP32 spectra
+    assert l2 > (1e-6 if prec in (PREC_BF16X3, PREC_FP16) else 1e-9)
 
 
 def test_uniform_gaussians_int8_digits_match_direct_sum(oracle_mod):
