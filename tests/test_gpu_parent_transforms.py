@@ -110,6 +110,33 @@ def test_scratch_in_rounds(extent, region):
 
 
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("region", [(1, 1, 1), None])
+def test_graphs_across_component_counts(region, precision):
+    """Solves of one, three and one component captured as graphs: each replay,
+    with other solves and growing work arrays in between, equals the eager result."""
+    print(f"case: graphs of one and three components, region {region}, precision {precision}", flush=True)
+    t = _uniform(10, region) if region else setups.VortexRings(
+        seed=7, block_extent=10, base_blocks=4, nref=2, nrings=3, centre_range=4.0, radius=(4.0, 8.0), core=(1.5, 2.5),
+        refinement_factor=0.5).tree
+    s, src, dst = _solver(t, precision, 3)
+    s.apply_lgf_batch(src, dst)
+    ref = [s.download(d) for d in dst]
+
+    def same(k):
+        return all(np.array_equal(s.download(d), x) for d, x in zip(dst[:k], ref))
+
+    s, src, dst = _solver(t, precision, 3)
+    s.set_graphs(True)
+    for k in (1, 1, 3, 1, 3, 1):
+        for d in dst:
+            s.upload(d, np.zeros(s.shape))
+        s.apply_lgf_batch(src[:k], dst[:k])
+        assert same(k), k
+        s.apply_lgf_batch(src, dst, kernel=1, alpha_base=0.3)  # grows the work arrays, before a solve does
+    s.set_graphs(False)
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
 def test_memory_of_a_component(precision):
     """A solve takes the memory of its work arrays, four fields and two
     block spectra of FP64 a component, and nothing beside them however its
