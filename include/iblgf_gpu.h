@@ -623,9 +623,10 @@ int iblgf_gpu_apply_lgf_typed(iblgf_gpu_ctx* ctx, int src_field, int dst_field, 
  *    array rounded up to 256 bytes: e.g. about 455 blocks at n = 10 in FP64)
  *    is refused with IBLGF_ERR_UNSUPPORTED.
  *  - The spectra of whole parents (the finest level's) lie in those spectra's
- *    part of the scratch.  Only meshes whose parents hold one or two blocks
- *    need more than it leaves; iblgf_gpu_prepare then puts an array aside
- *    (a few MB), which stays where it is until the context's tree is replaced.
+ *    part of the scratch.  Only trees whose parents hold one or two blocks, or
+ *    with few blocks above a large base level (FP32 spectra), need more than it
+ *    leaves; iblgf_gpu_prepare then puts an array aside (a few MB), which stays
+ *    where it is until the context's tree is replaced.
  *    So whatever other solves the context runs, the call allocates and frees
  *    nothing, and a graph that a caller captured around it stays valid until then.
  *  - All calls on one GPU share its scratch, which keeps the last call's

@@ -87,17 +87,25 @@ def _block():
     return t.init_refine(0).build_masks()
 
 
+def _thin():
+    """Few blocks at the finest level (64 of 874) above a base level of 512: with
+    FP32 spectra, the FP64 ones below the base level do not fit the region
+    beside the others either."""
+    return setups.VortexRings(seed=18, block_extent=6, base_blocks=8, nref=2, nrings=1, centre_range=9.0,
+                              radius=(0.3, 0.5), core=(0.6, 0.9), refinement_factor=0.96).tree
+
+
 def _free():
     torch.cuda.synchronize()
     return torch.cuda.mem_get_info()[0]
 
 
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
-@pytest.mark.parametrize("tree", ["rings", "uniform", "block"])
+@pytest.mark.parametrize("tree", ["rings", "uniform", "block", "thin"])
 def test_other_solves_between(tree, precision):
     print(f"case: noalloc between other solves, {tree}, precision {precision}", flush=True)
     t = {"rings": lambda: _rings(6).tree, "uniform": lambda: setups.UniformGaussians(seed=1000).tree,
-         "block": _block}[tree]()
+         "block": _block, "thin": _thin}[tree]()
     rng = np.random.default_rng(4)
     src = rng.standard_normal((t.info()["nblocks"],) + (t.n,) * 3)
     ref_solver = PoissonSolver(t)
