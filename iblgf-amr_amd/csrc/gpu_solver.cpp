@@ -1182,7 +1182,7 @@ const double2* GpuSolver::parent_ghat()
 // With FP32 spectra those below the base level are FP64 all the same: few
 // blocks, but the ones whose rounding reaches farthest.  In a 4290-block solve of
 // three components with FP32 spectra, 64 blocks of one level gave most of the
-// error: 9.1e-8, 5.2e-8, 1.6e-7 against FP64, 3.5e-8, 6.5e-8, 5.1e-8 with
+// error: 1.3e-7, 8.7e-8, 1.7e-7 against FP64, 3.5e-8, 6.5e-8, 5.1e-8 with
 // theirs in FP64, for 0.24 of 9.74 ms.
 GpuSolver::SpecPtrs GpuSolver::spectra(
     const PassPlan& p, int prec, const Batch& b, void* spec, size_t bytes, void* extra) const
